@@ -87,7 +87,7 @@ typedef struct lq_timing {
   double contract_ms;    /* moment contraction (Lᴴ R) incl. split-K reduce */
   double post_ms;        /* epilogues, Jackson, energy-grid sums */
   double spmv_bytes;     /* sum of 20*nnz + 4*(n+1) + (48 or 32)*k*n per launch */
-  double contract_flops; /* sum of 8*M0*M1*K per contraction */
+  double contract_flops; /* sum of 8*M0*M1*K per contraction (Kubo energy sums: of their transforms and products) */
   long long spmv_launches;
   long long contract_launches;
 } lq_timing;

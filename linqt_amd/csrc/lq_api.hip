@@ -846,6 +846,14 @@ int recursion_chunk_graph(lq_ctx ctx, const GraphKey &key, F &&body, hipGraphExe
 //   L_m = T_m(H~) OPL phi,  m < ML      (left recursion, src/chebyshev_moments.cpp:5-22)
 //   R^o_n = OPR_o T_n(H~) phi, n < MR   (right recursion + Multiply, src/chebyshev_vectors.cpp:24-51)
 // and accumulates raw_o += L^H R^o (K = n*g).
+// With sums set, the resident pipeline forms the Kubo energy sums' spectra from
+// the stored vectors in place of the tables (and says so in summed).
+struct KuboSums {
+  int formula;
+  const double2 *tables;
+  double2 *partial, *spec;
+};
+
 struct Pipe2D {
   lq_ctx ctx;
   lq_csr H, OPL;
@@ -854,6 +862,8 @@ struct Pipe2D {
   int n, ML, MR;
   double2 *raw;  // nopr tables of ML x MR (ld MR)
   int precision = LQ_PREC_FP64;
+  const KuboSums *sums = nullptr;
+  bool summed = false;
 };
 
 // out (+)= A^H B for A: MA rows (ld lda), B: MB rows (ld ldb), K columns, in
@@ -900,21 +910,47 @@ int contract_table(lq_ctx ctx, int precision, const double2 *A, long long lda, i
   return time_end(ctx, kCatPost, ev, 0);
 }
 
+// Elements between the stored vectors of consecutive orders: an odd number of
+// 128-byte lines.  Readers that walk over the orders at one site (the energy
+// sums) would otherwise meet the same memory channels again and again when
+// the vectors' length is a multiple of a large power of two: reading tiles of
+// 4 elements of all 1536 vectors of 2^21 took 17.1 ms for 51.5 GB (3.0 TB/s),
+// 11.9 ms (4.3 TB/s) with 9 more lines between them.
+size_t store_ld(size_t vec) { return ((vec + 7) / 8 | 1) * 8; }
+
+// The tables (or energy-sum spectra) of a group's stored vectors of K elements:
+// Ls [ML], Rs [nopr][MR], ld apart.
+int pipe2d_finish(Pipe2D &P, const double2 *Ls, const double2 *Rs, long long ld, long long K, bool accumulate) {
+  if (P.sums) {
+    hipEvent_t ev;
+    LQ_TRY(time_begin(P.ctx, kCatContract, &ev));
+    LQ_TRY(launch_kubosum(P.ctx->stream, P.sums->formula, Ls, Rs, ld, K, P.ML, P.nopr, P.sums->tables, P.sums->partial,
+                          P.sums->spec, accumulate ? 1 : 0));
+    P.summed = true;
+    return time_end(P.ctx, kCatContract, ev, kubosum_flops(P.ML, P.sums->formula, P.nopr, K));
+  }
+  // raw_o (+)= L^H R^o
+  for (int o = 0; o < P.nopr; ++o)
+    LQ_TRY(contract_table(P.ctx, P.precision, Ls, ld, P.ML, Rs + (size_t)o * P.MR * ld, ld, P.MR, K,
+                          P.raw + (size_t)o * P.ML * P.MR, P.MR, accumulate, o == 0));
+  return LQ_OK;
+}
+
 int pipe2d_group(Pipe2D &P, const double *phi, int r0, int g, bool accumulate) {
   lq_ctx ctx = P.ctx;
   const int n = P.n;
-  const size_t vec = (size_t)n * g;
+  const size_t vec = (size_t)n * g, ld = P.sums ? store_ld(vec) : vec;
   double2 *phi_d, *Ls, *Rw, *Rs;
   LQ_TRY(ctx_buf(ctx, "phi", vec * sizeof(double2), (void **)&phi_d));
-  LQ_TRY(ctx_buf(ctx, "Lstore", vec * (size_t)P.ML * sizeof(double2), (void **)&Ls));
+  LQ_TRY(ctx_buf(ctx, "Lstore", ld * (size_t)P.ML * sizeof(double2), (void **)&Ls));
   LQ_TRY(ctx_buf(ctx, "Rwork", 2 * vec * sizeof(double2), (void **)&Rw));
-  LQ_TRY(ctx_buf(ctx, "Rstore", vec * (size_t)P.MR * P.nopr * sizeof(double2), (void **)&Rs));
+  LQ_TRY(ctx_buf(ctx, "Rstore", ld * (size_t)P.MR * P.nopr * sizeof(double2), (void **)&Rs));
   LQ_TRY(upload_states(ctx, phi, n, r0, g, phi_d));
 
   const double2 one = d2(1, 0), zero = d2(0, 0), two = d2(2, 0), mone = d2(-1, 0);
   double2 *Rcur = Rw, *Rprev = Rw + vec;  // Rcur = T_n, Rprev = T_{n-1}
-  auto L = [&](int m) { return Ls + (size_t)m * vec; };
-  auto RS = [&](int o, int m) { return Rs + ((size_t)o * P.MR + m) * vec; };
+  auto L = [&](int m) { return Ls + (size_t)m * ld; };
+  auto RS = [&](int o, int m) { return Rs + ((size_t)o * P.MR + m) * ld; };
 
   SpmvLoopGuard guard{ctx};
   LQ_TRY(spmv_loop_begin(ctx));
@@ -975,10 +1011,7 @@ int pipe2d_group(Pipe2D &P, const double *phi, int r0, int g, bool accumulate) {
     // the last right slot, T_{MR-1}, is not the x of any step
     LQ_TRY(apply_opr(P.MR > 1 ? Rcur : Rprev, P.MR - 1));
     LQ_TRY(spmv_loop_end(ctx));
-    for (int o = 0; o < P.nopr; ++o)
-      LQ_TRY(contract_table(ctx, P.precision, Ls, (long long)vec, P.ML, RS(o, 0), (long long)vec, P.MR,
-                            (long long)vec, P.raw + (size_t)o * P.ML * P.MR, P.MR, accumulate, o == 0));
-    return LQ_OK;
+    return pipe2d_finish(P, Ls, Rs, (long long)ld, (long long)vec, accumulate);
   }
   if (P.MR > 0) LQ_TRY(apply_opr(Rprev, 0));
   // T1 = H~ T0 on both sides
@@ -1004,11 +1037,7 @@ int pipe2d_group(Pipe2D &P, const double *phi, int r0, int g, bool accumulate) {
     }
   }
   LQ_TRY(spmv_loop_end(ctx));
-  // raw_o (+)= L^H R^o
-  for (int o = 0; o < P.nopr; ++o)
-    LQ_TRY(contract_table(ctx, P.precision, Ls, (long long)vec, P.ML, RS(o, 0), (long long)vec, P.MR, (long long)vec,
-                          P.raw + (size_t)o * P.ML * P.MR, P.MR, accumulate, o == 0));
-  return LQ_OK;
+  return pipe2d_finish(P, Ls, Rs, (long long)ld, (long long)vec, accumulate);
 }
 
 // ---- the streamed 2D pipeline ------------------------------------------------
@@ -1367,6 +1396,24 @@ int run_pipe2d(Pipe2D &P, const double *phi, int R) {
     LQ_TRY(pipe2d_streamed(P, phi, r0, gg, r0 > 0, pl));
   }
   return LQ_OK;
+}
+
+// Kubo energy sums from transforms of the stored vectors (lq_kubosum.hip)
+// instead of the moment table.  Times at 262144 elements, Bastin, sums against
+// table (without the table's own energy sums, 6 M^2 flop at 70 TFLOP/s over
+// whole 128 x 128 tiles), one operator / two:
+//   M =  128: 1.27 / 1.68 ms against 0.37 / 0.74: up to there the table;
+//   M =  200: 1.41 / 1.84 against 1.47 / 2.95;  512: 2.56 / 3.39 against 5.9 / 11.8;
+//   M =  513 .. 640: 9.1 .. 10.1 / 11.3 .. 12.6 against 9.2 / 18.4 (three
+//   frequency sets that each read the vectors): the table for one operator;
+//   M =  700: 10.4 / 12.9 against 13.3 / 26.5;  1024: 15.4 / 19.9 against 23.6 / 47.
+// LQ_KUBO=table keeps the table.
+bool kubo_by_sums(int M, int nopr) {
+  static const bool off = [] {
+    const char *e = getenv("LQ_KUBO");
+    return e && strcmp(e, "table") == 0;
+  }();
+  return !off && M > 128 && (M <= 512 || M > 640 || nopr > 1) && kubosum_supported(M);
 }
 
 int ord_of(int p, int B) { return (p / B) * (B - 1) + (p % B); }
@@ -2242,32 +2289,49 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
     }
   }
   const size_t tab = (size_t)M * M;
-  double2 *raw, *fd;
+  double2 *raw, *fd, *tables = nullptr, *seq = nullptr;
   double *coef;
+  KuboSums sums{formula, nullptr, nullptr, nullptr};
+  const bool use_sums = precision == LQ_PREC_FP64 && kubo_by_sums(M, nopr);
   int rc = ctx_buf(ctx, "raw", tab * nopr * sizeof(double2), (void **)&raw);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_fd", (size_t)2 * nump * nopr * sizeof(double2), (void **)&fd);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_coef", (size_t)M * sizeof(double), (void **)&coef);
-  if (rc == LQ_OK) {
-    Pipe2D P{ctx, H, OPL, nopr, opr.data(), n, M, M, raw, precision};
-    rc = run_pipe2d(P, phi, R);
+  if (rc == LQ_OK && use_sums) {
+    const size_t count = kubosum_spec_count(M, formula, nopr);
+    rc = ctx_buf(ctx, "kubo_tables", kubosum_table_bytes(M), (void **)&tables);
+    if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_partial", kubosum_partial_bytes(M, formula), (void **)&sums.partial);
+    if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_spec", 2 * count * sizeof(double2), (void **)&sums.spec);
+    seq = sums.spec + count;
+    sums.tables = tables;
   }
+  // c_m = (2 - delta_m0) * Jackson_kernel(m, M) (src/Greenwood_FFTs.cpp:17-18)
+  std::vector<double> c(M);
+  for (int m = 0; m < M; ++m)
+    c[m] = (2 - (m == 0)) *
+           (1 / (M + 1.0) *
+            ((M - m + 1.0) * cos(kPi * m / (M + 1.0)) + sin(kPi * m / (M + 1.0)) / tan(kPi / (M + 1.0))));
+  hipError_t e = hipSuccess;
   if (rc == LQ_OK) {
-    // c_m = (2 - delta_m0) * Jackson_kernel(m, M) (src/Greenwood_FFTs.cpp:17-18)
-    std::vector<double> c(M);
-    for (int m = 0; m < M; ++m)
-      c[m] = (2 - (m == 0)) *
-             (1 / (M + 1.0) *
-              ((M - m + 1.0) * cos(kPi * m / (M + 1.0)) + sin(kPi * m / (M + 1.0)) / tan(kPi / (M + 1.0))));
-    hipError_t e = hipMemcpyAsync(coef, c.data(), sizeof(double) * M, hipMemcpyHostToDevice, ctx->stream);
+    e = hipMemcpyAsync(coef, c.data(), sizeof(double) * M, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess) {
       set_error("lq_kubo_fft: coefficient upload: %s", hipGetErrorString(e));
       rc = LQ_ERR_HIP;
     }
+  }
+  if (rc == LQ_OK && use_sums) rc = launch_kubosum_tables(ctx->stream, coef, M, tables);
+  Pipe2D P{ctx, H, OPL, nopr, opr.data(), n, M, M, raw, precision, use_sums ? &sums : nullptr};
+  if (rc == LQ_OK) rc = run_pipe2d(P, phi, R);
+  if (rc == LQ_OK) {
     hipEvent_t ev;
-    if (rc == LQ_OK) rc = time_begin(ctx, kCatPost, &ev);
-    if (rc == LQ_OK) rc = launch_scale(ctx->stream, raw, tab * nopr, 1.0 / R);
-    for (int o = 0; o < nopr && rc == LQ_OK; ++o)
-      rc = launch_kubo_pw(ctx->stream, raw + o * tab, M, M, nump, formula, coef, fd + (size_t)o * 2 * nump);
+    rc = time_begin(ctx, kCatPost, &ev);
+    if (P.summed) {
+      if (rc == LQ_OK)
+        rc = launch_kubosum_energies(ctx->stream, formula, sums.spec, tables, M, nopr, nump, 1.0 / R, seq, fd);
+    } else {
+      if (rc == LQ_OK) rc = launch_scale(ctx->stream, raw, tab * nopr, 1.0 / R);
+      for (int o = 0; o < nopr && rc == LQ_OK; ++o)
+        rc = launch_kubo_pw(ctx->stream, raw + o * tab, M, M, nump, formula, coef, fd + (size_t)o * 2 * nump);
+    }
     if (rc == LQ_OK) rc = time_end(ctx, kCatPost, ev, 0);
     if (rc == LQ_OK) {
       e = hipMemcpyAsync(final_data, fd, (size_t)2 * nump * nopr * sizeof(double2), hipMemcpyDeviceToHost, ctx->stream);

@@ -213,6 +213,23 @@ int split_nsplit(int M0, int M1, long long K);
 int launch_contract_split(hipStream_t st, int precision, const double2 *A, long long lda, int M0, const double2 *B,
                           long long ldb, int M1, long long K, double2 *work, int nsplit);
 
+// Kubo energy sums straight from the stored vectors (lq_kubosum.hip): L and
+// nopr right stores of [M] rows of K elements, ld apart, summed over K into the spectra spec
+// (kubosum_spec_count values, added to when accumulate != 0), then the 2 nump
+// energy sums per operator, scaled.  tables: kubosum_table_bytes, filled by
+// launch_kubosum_tables from the M damping coefficients; partial:
+// kubosum_partial_bytes; seq: as many values as spec.
+bool kubosum_supported(int M);
+size_t kubosum_table_bytes(int M);
+size_t kubosum_partial_bytes(int M, int formula);
+size_t kubosum_spec_count(int M, int formula, int nopr);
+double kubosum_flops(int M, int formula, int nopr, long long K);
+int launch_kubosum_tables(hipStream_t st, const double *coef, int M, double2 *tables);
+int launch_kubosum(hipStream_t st, int formula, const double2 *L, const double2 *R, long long ld, long long K, int M,
+                   int nopr, const double2 *tables, double2 *partial, double2 *spec, int accumulate);
+int launch_kubosum_energies(hipStream_t st, int formula, const double2 *spec, const double2 *tables, int M, int nopr,
+                            int nump, double scale, double2 *seq, double2 *out);
+
 // Post-processing (lq_post.hip).
 int launch_corr_epilogue(hipStream_t st, const double2 *raw, int ldr, const double2 *init, int M0,
                          int M1, int B, int R, double2 *out);
