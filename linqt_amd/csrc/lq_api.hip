@@ -2293,15 +2293,20 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
   double *coef;
   KuboSums sums{formula, nullptr, nullptr, nullptr};
   const bool use_sums = precision == LQ_PREC_FP64 && kubo_by_sums(M, nopr);
+  if (M > 4096) {
+    set_error("lq_kubo_fft: M = %d exceeds 4096", M);
+    for (auto m : owned) lq_csr_destroy(m);
+    return LQ_ERR_ARG;
+  }
+  const size_t count = kubosum_spec_count(M, formula, nopr);
   int rc = ctx_buf(ctx, "raw", tab * nopr * sizeof(double2), (void **)&raw);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_fd", (size_t)2 * nump * nopr * sizeof(double2), (void **)&fd);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_coef", (size_t)M * sizeof(double), (void **)&coef);
+  if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_seq", count * sizeof(double2), (void **)&seq);
   if (rc == LQ_OK && use_sums) {
-    const size_t count = kubosum_spec_count(M, formula, nopr);
     rc = ctx_buf(ctx, "kubo_tables", kubosum_table_bytes(M), (void **)&tables);
     if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_partial", kubosum_partial_bytes(M, formula), (void **)&sums.partial);
-    if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_spec", 2 * count * sizeof(double2), (void **)&sums.spec);
-    seq = sums.spec + count;
+    if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_spec", count * sizeof(double2), (void **)&sums.spec);
     sums.tables = tables;
   }
   // c_m = (2 - delta_m0) * Jackson_kernel(m, M) (src/Greenwood_FFTs.cpp:17-18)
@@ -2326,12 +2331,15 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
     rc = time_begin(ctx, kCatPost, &ev);
     if (P.summed) {
       if (rc == LQ_OK)
-        rc = launch_kubosum_energies(ctx->stream, formula, sums.spec, tables, M, nopr, nump, 1.0 / R, seq, fd);
+        rc = launch_kubosum_sequences(ctx->stream, formula, sums.spec, tables, M, nopr, 1.0 / R, seq);
     } else {
-      if (rc == LQ_OK) rc = launch_scale(ctx->stream, raw, tab * nopr, 1.0 / R);
+      double2 *diag;
+      if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_diag", diag_bytes(M, M), (void **)&diag);
       for (int o = 0; o < nopr && rc == LQ_OK; ++o)
-        rc = launch_kubo_pw(ctx->stream, raw + o * tab, M, M, nump, formula, coef, fd + (size_t)o * 2 * nump);
+        rc = launch_diag_kubo(ctx->stream, raw + o * tab, M, coef, formula, 1.0 / R, kubosum_length(M), diag,
+                              seq + o * (count / nopr));
     }
+    if (rc == LQ_OK) rc = launch_kubo_energies(ctx->stream, formula, seq, M, nopr, nump, fd);
     if (rc == LQ_OK) rc = time_end(ctx, kCatPost, ev, 0);
     if (rc == LQ_OK) {
       e = hipMemcpyAsync(final_data, fd, (size_t)2 * nump * nopr * sizeof(double2), hipMemcpyDeviceToHost, ctx->stream);
@@ -2639,15 +2647,16 @@ int lq_linear_grid(lq_ctx ctx, int kind, const double *mu, int M0, int M1, int n
   }
   if (kind == LQ_LIN_SPECTRAL) M1 = 1;
   DeviceGuard dg(ctx->device);
-  double2 *dm;
+  double2 *dm, *diag;
   double *kern, *dout;
   LQ_TRY(ctx_buf(ctx, "grid_mu", (size_t)M0 * M1 * sizeof(double2), (void **)&dm));
+  LQ_TRY(ctx_buf(ctx, "grid_diag", diag_bytes(M0, M1), (void **)&diag));
   LQ_TRY(ctx_buf(ctx, "grid_scratch", (size_t)2 * num_div * sizeof(double), (void **)&kern));
   LQ_TRY(ctx_buf(ctx, "grid_out", (size_t)2 * num_div * sizeof(double), (void **)&dout));
   LQ_HIP_CHECK(hipMemcpyAsync(dm, mu, (size_t)M0 * M1 * sizeof(double2), hipMemcpyHostToDevice, ctx->stream));
   hipEvent_t ev;
   LQ_TRY(time_begin(ctx, kCatPost, &ev));
-  LQ_TRY(launch_linear_grid(ctx->stream, kind, dm, M0, M1, n, W, Ec, num_div, kern, dout, dout + num_div));
+  LQ_TRY(launch_linear_grid(ctx->stream, kind, dm, M0, M1, n, W, Ec, num_div, diag, kern, dout, dout + num_div));
   LQ_TRY(time_end(ctx, kCatPost, ev, 0));
   const int rows = kind == LQ_LIN_SPECTRAL ? num_div : num_div - 1;
   LQ_HIP_CHECK(hipMemcpyAsync(E, dout, rows * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));

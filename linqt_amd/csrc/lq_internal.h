@@ -218,7 +218,8 @@ int launch_contract_split(hipStream_t st, int precision, const double2 *A, long 
 // (kubosum_spec_count values, added to when accumulate != 0), then the 2 nump
 // energy sums per operator, scaled.  tables: kubosum_table_bytes, filled by
 // launch_kubosum_tables from the M damping coefficients; partial:
-// kubosum_partial_bytes; seq: as many values as spec.
+// kubosum_partial_bytes; seq: as many values as spec.  launch_kubosum_sequences
+// takes the spectra back to the sequences.
 bool kubosum_supported(int M);
 size_t kubosum_table_bytes(int M);
 size_t kubosum_partial_bytes(int M, int formula);
@@ -227,15 +228,21 @@ double kubosum_flops(int M, int formula, int nopr, long long K);
 int launch_kubosum_tables(hipStream_t st, const double *coef, int M, double2 *tables);
 int launch_kubosum(hipStream_t st, int formula, const double2 *L, const double2 *R, long long ld, long long K, int M,
                    int nopr, const double2 *tables, double2 *partial, double2 *spec, int accumulate);
-int launch_kubosum_energies(hipStream_t st, int formula, const double2 *spec, const double2 *tables, int M, int nopr,
-                            int nump, double scale, double2 *seq, double2 *out);
+int launch_kubosum_sequences(hipStream_t st, int formula, const double2 *spec, const double2 *tables, int M, int nopr,
+                             double scale, double2 *seq);
+// The energy sums of nopr operators from their sequences A, B (and A' for
+// Bastin) of F = kubosum_length(M) values each.
+int kubosum_length(int M);
+int launch_kubo_energies(hipStream_t st, int formula, const double2 *seq, int M, int nopr, int nump, double2 *out);
 
 // Post-processing (lq_post.hip).
 int launch_corr_epilogue(hipStream_t st, const double2 *raw, int ldr, const double2 *init, int M0,
                          int M1, int B, int R, double2 *out);
-int launch_scale(hipStream_t st, double2 *x, size_t count, double s);
-int launch_kubo_pw(hipStream_t st, const double2 *mu, int ldm, int M, int nump, int formula,
-                   const double *coef, double2 *out);
+// Sums along a table's diagonals (lq_post.hip); diag: diag_bytes of scratch.
+// launch_diag_kubo: the sequences of launch_kubo_energies from a table (ld M).
+size_t diag_bytes(int M0, int M1);
+int launch_diag_kubo(hipStream_t st, const double2 *raw, int M, const double *coef, int formula, double scale, int F,
+                     double2 *diag, double2 *seq);
 int launch_kubo_post(hipStream_t st, int formula, const double2 *final_data, int nump, int n, double W,
                      double Ec, double *E, double *sigma, double *integrand);
 int launch_jackson_1d(hipStream_t st, double2 *mu, int maxMom);
@@ -255,7 +262,7 @@ int launch_timecorr_post(hipStream_t st, const double2 *mu, int M, int nT, int n
 // Linear-grid tools (kind = LQ_LIN_*): kern scratch of num_div doubles; E, out
 // receive num_div (spectral) or num_div - 1 rows.
 int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int M1, int n, double W, double Ec,
-                       int num_div, double *kern, double *E, double *out);
+                       int num_div, double2 *diag, double *kern, double *E, double *out);
 
 }  // namespace lq
 

@@ -536,11 +536,19 @@ int launch_kubosum(hipStream_t st, int formula, const double2 *L, const double2 
   return LQ_OK;
 }
 
-int launch_kubosum_energies(hipStream_t st, int formula, const double2 *spec, const double2 *tables, int M, int nopr,
-                            int nump, double scale, double2 *seq, double2 *out) {
-  const int H = sum_sets(M), F = kP * H, arr = sum_arrays(formula);
+int kubosum_length(int M) { return kP * sum_sets(M); }
+
+int launch_kubosum_sequences(hipStream_t st, int formula, const double2 *spec, const double2 *tables, int M, int nopr,
+                             double scale, double2 *seq) {
+  const int H = sum_sets(M), F = kP * H;
   const double2 *tf = tables + (size_t)H * kP * sum_fold(M) + kTw;
-  hipLaunchKernelGGL(k_sum_inverse, dim3(F, arr * nopr), dim3(64), 0, st, spec, F, tf, scale / F, seq);
+  hipLaunchKernelGGL(k_sum_inverse, dim3(F, sum_arrays(formula) * nopr), dim3(64), 0, st, spec, F, tf, scale / F, seq);
+  LQ_HIP_CHECK(hipGetLastError());
+  return LQ_OK;
+}
+
+int launch_kubo_energies(hipStream_t st, int formula, const double2 *seq, int M, int nopr, int nump, double2 *out) {
+  const int F = kubosum_length(M);
   if (formula == LQ_KUBO_BASTIN)
     hipLaunchKernelGGL((k_sum_energies<true>), dim3(nump, nopr), dim3(64), 0, st, seq, F, M, nump, out);
   else

@@ -2,6 +2,8 @@
 //
 // All FP64.  The single-thread sequential scans (cumulative integrals) keep
 // the reference's left-to-right summation order.
+#include <algorithm>
+
 #include "lq_internal.h"
 
 namespace lq {
@@ -50,88 +52,97 @@ __global__ void k_corr_epilogue(const double2 *__restrict__ raw, int ldr, const 
   out[t] = p <= q ? make_double2(tx, ty) : make_double2(tx, -ty);
 }
 
-__global__ void k_scale(double2 *__restrict__ x, long long count, double s) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < count) {
-    x[t].x *= s;
-    x[t].y *= s;
+// ---- sums along a table's diagonals -------------------------------------------
+// The energy-grid formulas weigh mu(m0, m1) by products of one factor in m0 and
+// one in m1 that are cosines, sines or e^{-i m theta}, some times m.  Such a
+// product depends on m0 + m1 and m1 - m0 only, so a formula at any number of
+// energies needs no more than the table's sums along its antidiagonals and
+// diagonals, O(M) terms per energy in place of O(M^2).  At M = 512 the 15360
+// energies of the linear-grid Bastin tool took 2.28 ms as a matrix-vector
+// product per energy (bound by re-reading the table from L2: 64 GB) and take
+// 0.05 ms for the sums and 0.07 ms for the energies; the 2048 energies of a
+// Kubo table 0.32 ms and now 0.06, 8e-16 from exact angles instead of 1e-14.
+//
+// part[chunk][4][Q], Q = M0 + M1 - 1, of the rows m0 of the chunk, index t:
+//   0: sum over m0 + m1 = t of v, 1: of w v, 2: over m1 - m0 = t - (M0 - 1) of v,
+//   3: of w v;  v = c[m0] c[m1] mu(m0, m1) (c null: 1), w = m0 or m1.
+// Thread t reads one element of each row, consecutive threads consecutive ones.
+__global__ __launch_bounds__(64) void k_diag_sums(const double2 *__restrict__ mu, int ld, int M0, int M1, int rows,
+                                                  const double *__restrict__ c, int weight_m1,
+                                                  double2 *__restrict__ part) {
+  const int Q = M0 + M1 - 1;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int r0 = blockIdx.y * rows, r1 = min(M0, r0 + rows);
+  if (t >= Q) return;
+  double2 a = make_double2(0.0, 0.0), a1 = a, b = a, b1 = a;
+  auto add = [&](double2 &s, double2 &s1, int m0, int m1) {
+    if (m1 < 0 || m1 >= M1) return;
+    double2 v = mu[(size_t)m0 * ld + m1];
+    if (c) {
+      const double f = c[m0] * c[m1];
+      v.x *= f;
+      v.y *= f;
+    }
+    const double w = weight_m1 ? m1 : m0;
+    s.x += v.x;
+    s.y += v.y;
+    s1.x = fma(w, v.x, s1.x);
+    s1.y = fma(w, v.y, s1.y);
+  };
+#pragma unroll 4
+  for (int m0 = r0; m0 < r1; ++m0) {
+    add(a, a1, m0, t - m0);
+    add(b, b1, m0, t - (M0 - 1) + m0);
+  }
+  double2 *o = part + (size_t)blockIdx.y * 4 * Q + t;
+  o[0] = a;
+  o[Q] = a1;
+  o[2 * (size_t)Q] = b;
+  o[3 * (size_t)Q] = b1;
+}
+
+__device__ __forceinline__ double2 diag_sum(const double2 *__restrict__ part, int nchunk, int Q, int which, int t) {
+  double2 v = make_double2(0.0, 0.0);
+  for (int c = 0; c < nchunk; ++c) {
+    const double2 p = part[((size_t)c * 4 + which) * Q + t];
+    v.x += p.x;
+    v.y += p.y;
+  }
+  return v;
+}
+
+// Sequences of a Kubo table for launch_kubo_energies, scaled: A at 0, B at F
+// (B_q at index q mod F) and, with deriv, A' at 2 F.
+__global__ __launch_bounds__(64) void k_diag_kubo(const double2 *__restrict__ part, int nchunk, int M, int F, int deriv,
+                                                  double scale, double2 *__restrict__ seq) {
+  const int Q = 2 * M - 1, t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= Q) return;
+  const double2 a = diag_sum(part, nchunk, Q, 0, t), b = diag_sum(part, nchunk, Q, 2, t);
+  const int q = t - (M - 1);
+  seq[t] = make_double2(scale * a.x, scale * a.y);
+  seq[F + (q < 0 ? q + F : q)] = make_double2(scale * b.x, scale * b.y);
+  if (deriv) {
+    const double2 d = diag_sum(part, nchunk, Q, 1, t);
+    seq[2 * F + t] = make_double2(scale * d.x, scale * d.y);
   }
 }
 
-// Per-energy sums of Kubo_solver_FFT's per-site DFT products
-// (src/Greenwood_FFTs.cpp:59-83, src/Bastin_FFTs.cpp:172-257) written through
-// the moment table mu(m, n) = <L_m|R_n> (mean over states):
-//   theta_k = pi (2k + 1/2) / nump, s = +1 for k < nump/2 else -1,
-//   t_m = c_m cos(m theta), e_m = c_m exp(i s m theta), d_m = m e_m,
-//   Greenwood: r_k = Re sum t_m t_n mu_mn
-//   Bastin:    p_k = sum mu_mn (t_m e_n + conj(e_m) t_n)
-//              w_k = sum mu_mn (conj(d_m) t_n - t_m d_n)
-// with c_m = (2 - delta_m0) g_m (Jackson, Kubo_solver_FFT.hpp:99-107).
-// One block per energy; thread j owns columns n = j, j+256, ...
-__global__ __launch_bounds__(256) void k_kubo_pw(const double2 *__restrict__ mu, int ldm, int M, int nump,
-                                                 int formula, const double *__restrict__ coef,
-                                                 double2 *__restrict__ out) {
-  extern __shared__ double tab[];  // [3*M]: t_m, e_m (re, im) -> (c cos, c sin)
-  double *tc = tab, *ts = tab + M;
-  const int k = blockIdx.x;
-  const double theta = kPi * (2 * k + 0.5) / nump;
-  const double sgn = (k < nump / 2) ? 1.0 : -1.0;
-  for (int m = threadIdx.x; m < M; m += blockDim.x) {
-    double sn, cs;
-    sincos(m * theta, &sn, &cs);
-    tc[m] = coef[m] * cs;
-    ts[m] = coef[m] * sgn * sn;
-  }
-  __syncthreads();
-  double pr = 0, pi = 0, wr = 0, wi = 0, rr = 0;
-  for (int nn = threadIdx.x; nn < M; nn += blockDim.x) {
-    // z^t = sum_m t_m mu_mn ; z^e = sum_m conj(e_m) mu_mn ; z^d = sum_m m conj(e_m) mu_mn
-    double ztr = 0, zti = 0, zer = 0, zei = 0, zdr = 0, zdi = 0;
-    for (int m = 0; m < M; ++m) {
-      const double2 a = mu[(size_t)m * ldm + nn];
-      const double t = tc[m], er = tc[m], ei = -ts[m];  // conj(e_m) = c cos - i c s sin
-      ztr = fma(t, a.x, ztr);
-      zti = fma(t, a.y, zti);
-      const double cr = er * a.x - ei * a.y, ci = er * a.y + ei * a.x;
-      zer += cr;
-      zei += ci;
-      zdr = fma((double)m, cr, zdr);
-      zdi = fma((double)m, ci, zdi);
-    }
-    const double tn = tc[nn], enr = tc[nn], eni = ts[nn];
-    if (formula == LQ_KUBO_GREENWOOD) {
-      rr += tn * ztr;
-    } else {
-      const double dnr = nn * enr, dni = nn * eni;
-      // p += z^t * e_n + z^e * t_n
-      pr += ztr * enr - zti * eni + zer * tn;
-      pi += ztr * eni + zti * enr + zei * tn;
-      // w += z^d * t_n - z^t * d_n
-      wr += zdr * tn - (ztr * dnr - zti * dni);
-      wi += zdi * tn - (ztr * dni + zti * dnr);
-    }
-  }
-  __shared__ double red[5][256];
-  red[0][threadIdx.x] = pr;
-  red[1][threadIdx.x] = pi;
-  red[2][threadIdx.x] = wr;
-  red[3][threadIdx.x] = wi;
-  red[4][threadIdx.x] = rr;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-      for (int q = 0; q < 5; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    if (formula == LQ_KUBO_GREENWOOD) {
-      out[k] = make_double2(red[4][0], 0.0);
-      out[k + nump] = make_double2(0.0, 0.0);
-    } else {
-      out[k] = make_double2(red[0][0], red[1][0]);
-      out[k + nump] = make_double2(red[2][0], red[3][0]);
-    }
-  }
+// U_q for q >= 0, interleaved [Q][4], of the grid tools (weight m1):
+//   0: Re, even in q:  (A_q + B_q + B_-q) / 2,     1: Im, odd:  (A_q + B_q - B_-q) / 2,
+//   2: Im, even, of the weighted sums,             3: Re, odd, of the weighted sums.
+__global__ __launch_bounds__(64) void k_diag_grid(const double2 *__restrict__ part, int nchunk, int M0, int M1,
+                                                  double *__restrict__ seq) {
+  const int Q = M0 + M1 - 1, q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= Q) return;
+  const double2 z = make_double2(0.0, 0.0);
+  const double2 a = diag_sum(part, nchunk, Q, 0, q), a1 = diag_sum(part, nchunk, Q, 1, q);
+  const bool p = q <= M1 - 1, m = q > 0 && q <= M0 - 1;
+  const double2 bp = p ? diag_sum(part, nchunk, Q, 2, M0 - 1 + q) : z, bp1 = p ? diag_sum(part, nchunk, Q, 3, M0 - 1 + q) : z;
+  const double2 bm = m ? diag_sum(part, nchunk, Q, 2, M0 - 1 - q) : z, bm1 = m ? diag_sum(part, nchunk, Q, 3, M0 - 1 - q) : z;
+  seq[4 * q] = 0.5 * (a.x + bp.x + bm.x);
+  seq[4 * q + 1] = 0.5 * (a.y + bp.y - bm.y);
+  seq[4 * q + 2] = 0.5 * (a1.y + bp1.y + bm1.y);
+  seq[4 * q + 3] = 0.5 * (a1.x + bp1.x - bm1.x);
 }
 
 // rearrange_crescent_order (src/Kubo_solver_FFT_postProcess.cpp:98-116) as an
@@ -148,40 +159,73 @@ __device__ __forceinline__ int crescent_src(int j, int nump) {
   return i;
 }
 
+// out(i) = sum of term(j), j <= i, for i < n, by one block of 256 threads in the
+// reference's order, left to right: the terms of a chunk are formed by all
+// threads, added up by thread 0, and stored by all.  15360 terms read, added and
+// stored by one thread took 3.65 ms (a memory round trip each); 0.19 ms here,
+// where the chain of dependent additions is what is left.
+constexpr int kScan = 2048;
+template <class Term, class Store>
+__device__ void ordered_sums(int n, Term term, Store store) {
+  __shared__ double sh[kScan];
+  const int tid = threadIdx.x;
+  double acc = 0.0;
+  for (int base = 0; base < n; base += kScan) {
+    const int len = min(kScan, n - base);
+    for (int i = tid; i < kScan; i += 256) sh[i] = i < len ? term(base + i) : 0.0;
+    __syncthreads();
+    if (tid == 0) {
+      for (int i = 0; i < len; i += 16) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = sh[i + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = acc += v[u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) sh[i + u] = v[u];
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < len; i += 256) store(base + i, sh[i]);
+    __syncthreads();
+  }
+}
+
 // Kubo_solver_FFT_postProcess (src/Kubo_solver_FFT_postProcess.cpp:8-16, 36-47,
-// 120-273, 279-397), one block; the cumulative sum runs on one thread.
-__global__ void k_kubo_post(int formula, const double2 *__restrict__ fd, int nump, int n, double W, double Ec,
-                            double *__restrict__ Eo, double *__restrict__ so, double *__restrict__ integ) {
+// 120-273, 279-397): the columns of each energy; Bastin's cumulative sum in
+// k_kubo_post_sums.
+__device__ __forceinline__ double kubo_energy(int j, int nump) {
+  return cos(kPi * (2 * crescent_src(j, nump) + 0.5) / nump);
+}
+
+__global__ __launch_bounds__(64) void k_kubo_post(int formula, const double2 *__restrict__ fd, int nump, int n, double W,
+                                                  double Ec, double *__restrict__ Eo, double *__restrict__ so,
+                                                  double *__restrict__ integ) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= nump) return;
   const double a = W / 2.0, b = Ec;
   const double omega = n / (a * a);
-  for (int j = threadIdx.x; j < nump; j += blockDim.x) {
-    const int k = crescent_src(j, nump);
-    const double e = cos(kPi * (2 * k + 0.5) / nump);
-    Eo[j] = a * e - b;
-    if (formula == LQ_KUBO_BASTIN) {
-      double v = e * fd[k].x - (sqrt(1.0 - e * e) * fd[k + nump].y);
-      v *= 1.0 / pow((1.0 - e * e), 2.0);
-      v *= omega / (kPi);
-      integ[j] = v;
-    } else {
-      so[j] = 2.0 * omega * fd[k].x / (1.0 - e * e) / (2 * kPi);
-      if (integ) integ[j] = 0.0;
-    }
+  const int k = crescent_src(j, nump);
+  const double e = kubo_energy(j, nump);
+  Eo[j] = a * e - b;
+  if (formula == LQ_KUBO_BASTIN) {
+    double v = e * fd[k].x - (sqrt(1.0 - e * e) * fd[k + nump].y);
+    v *= 1.0 / pow((1.0 - e * e), 2.0);
+    v *= omega / (kPi);
+    integ[j] = v;
+  } else {
+    so[j] = 2.0 * omega * fd[k].x / (1.0 - e * e) / (2 * kPi);
+    if (integ) integ[j] = 0.0;
   }
-  if (formula != LQ_KUBO_BASTIN) return;
-  // ascending energies in LDS, then the left-Riemann cumulative sum in the
-  // reference's order on one thread
-  extern __shared__ double er[];
-  for (int j = threadIdx.x; j < nump; j += blockDim.x) er[j] = cos(kPi * (2 * crescent_src(j, nump) + 0.5) / nump);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double acc = 0;
-    for (int i = 0; i < nump - 1; ++i) {
-      acc += integ[i] * (er[i + 1] - er[i]);
-      so[i] = acc;
-    }
-    so[nump - 1] = 0.0;
-  }
+}
+
+// ascending energies, left-Riemann cumulative sum
+__global__ __launch_bounds__(256) void k_kubo_post_sums(int nump, const double *__restrict__ integ,
+                                                        double *__restrict__ so) {
+  ordered_sums(
+      nump - 1, [&](int i) { return integ[i] * (kubo_energy(i + 1, nump) - kubo_energy(i, nump)); },
+      [&](int i, double v) { so[i] = v; });
+  if (threadIdx.x == 0) so[nump - 1] = 0.0;
 }
 
 // Moments1D::ApplyJacksonKernel (src/chebyshev_moments1D.cpp:79-86).
@@ -265,6 +309,10 @@ __global__ __launch_bounds__(64) void k_dos_fftgrid(const double2 *__restrict__ 
 // kuboGreenwoodFromChebmom_FFTgrid.cpp:57-66 and kuboBastinFromChebmom_FFTgrid.cpp:77-86:
 // one block per energy; thread j owns columns m1 = j, j+256, ...:
 //   kernel = sum_m1 Im( G(E, m1) * sum_m0 delta(E, m0) mu(m0, m1) ).
+// Not through the table's diagonal sums: these grids go up to the band edges,
+// where the sum over m0 cancels and 1/f^4 magnifies what is left of it; from
+// the diagonal sums the Bastin curve at M = 512 was 1.3e-10 off instead of 9e-12
+// (0.13 ms against 0.09).
 template <int DERIV>
 __global__ __launch_bounds__(256) void k_grid2d(const double2 *__restrict__ mu, int M0, int M1, const double *__restrict__ energies,
                                                 double *__restrict__ kern) {
@@ -294,22 +342,25 @@ __global__ __launch_bounds__(256) void k_grid2d(const double2 *__restrict__ mu, 
   if (threadIdx.x == 0) kern[i] = red[0];
 }
 
-// Linear-grid tools (src/*FromChebmom.cpp), kinds as LQ_LIN_*: one block per
-// energy evaluates the tool's double sum in separable form,
-//   sum_m1 proj( b_m1(x) * sum_m0 a_m0(x) mu(m0, m1) ),
-// with (a, b, proj) = (delta, gR, Im) Greenwood/BastinI, (delta, DgR, Im)
-// Bastin, (delta, delta, Re) Surf, (Im gR, Re DgR, 4 Im) Sea; BastinII uses
-// the two left vectors gR and DgR: -Re(DgR_m1 z_gR - gR_m1 z_DgR).
+// Linear-grid tools (src/*FromChebmom.cpp), kinds as LQ_LIN_*.  Every tool's
+// double sum is sum_m1 proj( b_m1(x) * sum_m0 a_m0(x) mu(m0, m1) ) with
+// (a, b, proj) = (delta, gR, Im) Greenwood/BastinI, (delta, DgR, Im) Bastin,
+// (delta, delta, Re) Surf, (Im gR, Re DgR, 4 Im) Sea; BastinII uses the two left
+// vectors gR and DgR: -Re(DgR_m1 z_gR - gR_m1 z_DgR).
 __device__ __forceinline__ double lin_xgrid(int kind, int i, int num_div) {
   const double xb = kind == 2 ? 0.99 : 1.0;
   return -xb + i * (2 * xb) / (num_div - 1);
 }
 
+// One block per energy i = step * block, the sums as written above.  step = 1,
+// every energy: Spectral, BastinII and small tables.  step = num_div - 1, the two
+// end points of the others, where x = +-1 makes every coefficient infinite and
+// the printed NaN or infinity is the one the sources' order of operations gives.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1, int num_div,
-                                                       double scale, double *__restrict__ kern) {
+                                                       int step, double scale, double *__restrict__ kern) {
   extern __shared__ double2 lv[];  // left vector(s): [M0] (BastinII: [2][M0])
-  const int i = blockIdx.x;
+  const int i = blockIdx.x * step;
   const double x = lin_xgrid(KIND, i, num_div);
   for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) {
     if (KIND == 4) {
@@ -368,29 +419,102 @@ __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict
   if (threadIdx.x == 0) kern[i] = red[0] * scale;
 }
 
-// The printed columns, in the sources' left-to-right order (one thread: the
-// running sums must keep that order).
-__global__ void k_linear_finish(int kind, int num_div, double a, double Ec, const double *__restrict__ kern,
-                                double *__restrict__ E, double *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const int rows = kind == 0 ? num_div : num_div - 1;
-  double acc = 0;
-  for (int i = 0; i < rows; ++i) {
-    const double x = lin_xgrid(kind, i, num_div);
-    E[i] = x * a + Ec;
-    if (kind == 0 || kind == 1) {
-      out[i] = kern[i];
-    } else {
-      const double dx = lin_xgrid(kind, i + 1, num_div) - x;
-      switch (kind) {
-        case 2: acc += kern[i] * dx; out[i] = acc; break;
-        case 3: out[i] = 0.5 * (kern[i] + kern[i + 1]); break;
-        case 4: acc += (kern[i] + kern[i + 1]) * dx; out[i] = acc; break;
-        case 5: acc += 0.5 * (kern[i] + kern[i + 1]) * dx; out[i] = acc; break;
-        default: out[i] = (kern[i + 1] + kern[i]) / 2.0; break;
+// The same sums through the table's diagonal sums U (k_diag_grid): with
+// theta = acos x, f = sin theta,
+//   C1 = sum cos m0 cos m1 Re mu = sum_q U0 cos q theta,  S1 = sum cos m0 sin m1 Im mu = sum U1 sin,
+//   C2 = sum m1 cos m0 cos m1 Im mu = sum U2 cos,         S2 = sum m1 cos m0 sin m1 Re mu = sum U3 sin,
+//   Greenwood, BastinI  -(C1 + S1) / (pi f^2);   Surf  C1 / (pi f)^2;
+//   Bastin  [f (C2 - S2) - x (C1 + S1)] / (pi f^4);  Sea  -4 [f C2 - x S1] / f^4.
+// One wavefront for kEw energies (the U of a lane's q are loaded once for all).
+// The angle is taken from the nearer band edge, theta' = acos |x|, with the
+// parity of q for x < 0: the phases' rounding q theta' 2^-53 then is smallest
+// towards the edges, where 1/f^4 magnifies it.
+constexpr int kEw = 4;
+template <int KIND>
+__global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__ seq, int Q,
+                                                      int num_div, double scale, double *__restrict__ kern) {
+  const int l = threadIdx.x, i0 = blockIdx.x * kEw;
+  double x[kEw], th[kEw], u[kEw], v[kEw];
+#pragma unroll
+  for (int e = 0; e < kEw; ++e) {
+    const int i = min(i0 + e, num_div - 1);
+    x[e] = lin_xgrid(KIND, i, num_div);
+    th[e] = acos(fabs(x[e]));
+    u[e] = v[e] = 0.0;
+  }
+  for (int q = l; q < Q; q += 64) {
+    const double4 w = *(const double4 *)(seq + 4 * (size_t)q);
+#pragma unroll
+    for (int e = 0; e < kEw; ++e) {
+      double sn, cs;
+      sincos(q * th[e], &sn, &cs);
+      if (x[e] < 0.0) {  // q theta = q pi - q theta'
+        if (q & 1)
+          cs = -cs;
+        else
+          sn = -sn;
+      }
+      // u: the sum without the weight m1, v: the weighted one
+      if (KIND == 6) {
+        u[e] = fma(w.x, cs, u[e]);
+      } else if (KIND == 5) {
+        u[e] = fma(w.y, sn, u[e]);
+        v[e] = fma(w.z, cs, v[e]);
+      } else {
+        u[e] = fma(w.x, cs, fma(w.y, sn, u[e]));
+        if (KIND == 2) v[e] = fma(w.z, cs, fma(-w.w, sn, v[e]));
       }
     }
   }
+#pragma unroll
+  for (int e = 0; e < kEw; ++e) {
+    for (int d = 32; d > 0; d >>= 1) {
+      u[e] += __shfl_down(u[e], d);
+      v[e] += __shfl_down(v[e], d);
+    }
+    const int i = i0 + e;
+    // the linear grid's end points belong to k_linear_kernel (x = +-1; not Bastin's)
+    const bool end = KIND != 2 && (i == 0 || i == num_div - 1);
+    if (l == 0 && i < num_div && !end) {
+      const double f2 = 1.0 - x[e] * x[e], f = sqrt(f2);
+      double r;
+      if (KIND == 6)
+        r = u[e] / f2 / (kPi * kPi);
+      else if (KIND == 5)
+        r = -4.0 * (f * v[e] - x[e] * u[e]) / f2 / f2;
+      else if (KIND == 2)
+        r = (f * v[e] - x[e] * u[e]) / f2 / f2 / kPi;
+      else
+        r = -u[e] / f2 / kPi;
+      kern[i] = r * scale;
+    }
+  }
+}
+
+// The printed columns: E and the values that need no running sum.
+__global__ __launch_bounds__(64) void k_linear_columns(int kind, int num_div, double a, double Ec,
+                                                       const double *__restrict__ kern, double *__restrict__ E,
+                                                       double *__restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (kind == 0 ? num_div : num_div - 1)) return;
+  E[i] = lin_xgrid(kind, i, num_div) * a + Ec;
+  switch (kind) {
+    case 0: case 1: out[i] = kern[i]; break;
+    case 3: out[i] = 0.5 * (kern[i] + kern[i + 1]); break;
+    case 6: out[i] = (kern[i + 1] + kern[i]) / 2.0; break;
+    default: break;  // k_linear_sums
+  }
+}
+
+__global__ __launch_bounds__(256) void k_linear_sums(int kind, int num_div, const double *__restrict__ kern,
+                                                     double *__restrict__ out) {
+  ordered_sums(
+      num_div - 1,
+      [&](int i) {
+        const double dx = lin_xgrid(kind, i + 1, num_div) - lin_xgrid(kind, i, num_div);
+        return kind == 2 ? kern[i] * dx : kind == 4 ? (kern[i] + kern[i + 1]) * dx : 0.5 * (kern[i] + kern[i + 1]) * dx;
+      },
+      [&](int i, double v) { out[i] = v; });
 }
 
 // y (=|+=) c x over count complex elements (Bessel-Chebyshev time evolution).
@@ -450,23 +574,68 @@ __global__ void k_greenwood_finish(int num_div, int n, double W, double Ec, cons
   out[i] = -1.0 * kern[i] * (n / a / a);
 }
 
-__global__ void k_bastin_finish(int num_div, int n, double W, double Ec, const double *__restrict__ energies,
-                                double *__restrict__ kern, double *__restrict__ E, double *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(256) void k_bastin_finish(int num_div, int n, double W, double Ec,
+                                                       const double *__restrict__ energies,
+                                                       const double *__restrict__ kern, double *__restrict__ E,
+                                                       double *__restrict__ out) {
   const double a = W / 2.0;
-  double acc = 0;
-  for (int i = 0; i < num_div - 1; ++i) {
-    const double k = kern[i] * (-2.0 * n / a / a);
-    acc += k * (energies[i + 1] - energies[i]);
-    E[i] = energies[i] * a + Ec;
-    out[i] = acc;
+  for (int i = threadIdx.x; i < num_div - 1; i += 256) E[i] = energies[i] * a + Ec;
+  ordered_sums(
+      num_div - 1, [&](int i) { return kern[i] * (-2.0 * n / a / a) * (energies[i + 1] - energies[i]); },
+      [&](int i, double v) { out[i] = v; });
+}
+
+// Rows of a table summed by one block of k_diag_sums: enough blocks for the
+// chip at M = 512 (16 x 16), at most 64 partial sums of a diagonal.
+int diag_rows(int M0) { return std::max(32, (M0 + 63) / 64); }
+int diag_chunks(int M0) { return (M0 + diag_rows(M0) - 1) / diag_rows(M0); }
+
+int launch_diag_sums(hipStream_t st, const double2 *mu, int ld, int M0, int M1, const double *c, int weight_m1,
+                     double2 *part) {
+  const int Q = M0 + M1 - 1, rows = diag_rows(M0);
+  hipLaunchKernelGGL(k_diag_sums, dim3((Q + 63) / 64, diag_chunks(M0)), dim3(64), 0, st, mu, ld, M0, M1, rows, c,
+                     weight_m1, part);
+  LQ_HIP_CHECK(hipGetLastError());
+  return LQ_OK;
+}
+
+// kern[i] of a grid tool (kinds as k_grid_energies) from the table's diagonal sums.
+int launch_grid_kernel(hipStream_t st, int kind, const double2 *mu, int M0, int M1, int num_div, double scale,
+                       double2 *diag, double *kern) {
+  const int Q = M0 + M1 - 1;
+  LQ_TRY(launch_diag_sums(st, mu, M1, M0, M1, nullptr, 1, diag));
+  double *seq = (double *)(diag + (size_t)4 * Q * diag_chunks(M0));
+  hipLaunchKernelGGL(k_diag_grid, dim3((Q + 63) / 64), dim3(64), 0, st, diag, diag_chunks(M0), M0, M1, seq);
+  const dim3 grid((num_div + kEw - 1) / kEw);
+  switch (kind) {
+#define LQ_GE(K) \
+  case K: hipLaunchKernelGGL((k_grid_energies<K>), grid, dim3(64), 0, st, seq, Q, num_div, scale, kern); break;
+    LQ_GE(1) LQ_GE(2) LQ_GE(5) LQ_GE(6)
+    case 3: hipLaunchKernelGGL((k_grid_energies<1>), grid, dim3(64), 0, st, seq, Q, num_div, scale, kern); break;
+#undef LQ_GE
   }
+  LQ_HIP_CHECK(hipGetLastError());
+  return LQ_OK;
 }
 
 }  // namespace
 
+size_t diag_bytes(int M0, int M1) {
+  return sizeof(double2) * (size_t)4 * (M0 + M1 - 1) * diag_chunks(M0) + 4 * sizeof(double) * (size_t)(M0 + M1 - 1);
+}
+
+int launch_diag_kubo(hipStream_t st, const double2 *raw, int M, const double *coef, int formula, double scale, int F,
+                     double2 *diag, double2 *seq) {
+  const int Q = 2 * M - 1;
+  LQ_TRY(launch_diag_sums(st, raw, M, M, M, coef, 0, diag));
+  hipLaunchKernelGGL(k_diag_kubo, dim3((Q + 63) / 64), dim3(64), 0, st, diag, diag_chunks(M), M, F,
+                     formula == LQ_KUBO_BASTIN ? 1 : 0, scale, seq);
+  LQ_HIP_CHECK(hipGetLastError());
+  return LQ_OK;
+}
+
 int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int M1, int n, double W, double Ec,
-                       int num_div, double *kern, double *E, double *out) {
+                       int num_div, double2 *diag, double *kern, double *E, double *out) {
   const double a = W / 2.0;
   double scale;
   switch (kind) {
@@ -484,13 +653,28 @@ int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int 
     set_error("launch_linear_grid: %d moments exceed the LDS table (max %d)", M0, kind == 4 ? 2048 : 4096);
     return LQ_ERR_UNSUPPORTED;
   }
+  // Through the diagonal sums from 64 x 64 moments on: 0.12 ms instead of 2.28 at
+  // M = 512 (15360 energies), and there 4e-14 from exact sums instead of 3e-13;
+  // below, the direct sums take a few microseconds and are as near (M = 40 x 65,
+  // Bastin: 8e-15 instead of 2e-14).
+  const bool diagonal = kind != 0 && kind != 4 && (long long)M0 * M1 >= 4096;
+  auto direct = [&](auto kernel) {
+    const bool ends = diagonal;
+    hipLaunchKernelGGL(kernel, dim3(ends ? 2 : num_div), dim3(256), lds, st, mu, M0, M1, num_div,
+                       ends ? num_div - 1 : 1, scale, kern);
+  };
+  if (diagonal) LQ_TRY(launch_grid_kernel(st, kind, mu, M0, M1, num_div, scale, diag, kern));
   switch (kind) {
-#define LQ_LIN(K) \
-  case K: hipLaunchKernelGGL((k_linear_kernel<K>), dim3(num_div), dim3(256), lds, st, mu, M0, M1, num_div, scale, kern); break;
-    LQ_LIN(0) LQ_LIN(1) LQ_LIN(2) LQ_LIN(3) LQ_LIN(4) LQ_LIN(5) LQ_LIN(6)
-#undef LQ_LIN
+    case 0: direct(k_linear_kernel<0>); break;
+    case 1: case 3: direct(k_linear_kernel<1>); break;
+    case 2: if (!diagonal) direct(k_linear_kernel<2>); break;  // its grid ends inside (-1, 1)
+    case 4: direct(k_linear_kernel<4>); break;
+    case 5: direct(k_linear_kernel<5>); break;
+    case 6: direct(k_linear_kernel<6>); break;
   }
-  hipLaunchKernelGGL(k_linear_finish, dim3(1), dim3(64), 0, st, kind, num_div, a, Ec, kern, E, out);
+  hipLaunchKernelGGL(k_linear_columns, dim3((num_div + 63) / 64), dim3(64), 0, st, kind, num_div, a, Ec, kern, E, out);
+  if (kind == 2 || kind == 4 || kind == 5)
+    hipLaunchKernelGGL(k_linear_sums, dim3(1), dim3(256), 0, st, kind, num_div, kern, out);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }
@@ -527,33 +711,16 @@ int launch_corr_epilogue(hipStream_t st, const double2 *raw, int ldr, const doub
   return LQ_OK;
 }
 
-int launch_scale(hipStream_t st, double2 *x, size_t count, double s) {
-  if (count == 0) return LQ_OK;
-  hipLaunchKernelGGL(k_scale, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, x, (long long)count, s);
-  LQ_HIP_CHECK(hipGetLastError());
-  return LQ_OK;
-}
-
-int launch_kubo_pw(hipStream_t st, const double2 *mu, int ldm, int M, int nump, int formula, const double *coef,
-                   double2 *out) {
-  const size_t lds = sizeof(double) * 2 * (size_t)M;
-  if (lds > 64 * 1024) {
-    set_error("kubo_pw: M = %d exceeds the LDS table limit (4096)", M);
-    return LQ_ERR_ARG;
-  }
-  hipLaunchKernelGGL(k_kubo_pw, dim3(nump), dim3(256), lds, st, mu, ldm, M, nump, formula, coef, out);
-  LQ_HIP_CHECK(hipGetLastError());
-  return LQ_OK;
-}
-
 int launch_kubo_post(hipStream_t st, int formula, const double2 *final_data, int nump, int n, double W, double Ec,
                      double *E, double *sigma, double *integrand) {
   if ((size_t)nump * sizeof(double) > 64 * 1024) {
     set_error("kubo_post: nump = %d exceeds 8192", nump);
     return LQ_ERR_ARG;
   }
-  hipLaunchKernelGGL(k_kubo_post, dim3(1), dim3(256), (size_t)nump * sizeof(double), st, formula, final_data, nump, n,
-                     W, Ec, E, sigma, integrand);
+  hipLaunchKernelGGL(k_kubo_post, dim3((nump + 63) / 64), dim3(64), 0, st, formula, final_data, nump, n, W, Ec, E, sigma,
+                     integrand);
+  if (formula == LQ_KUBO_BASTIN)
+    hipLaunchKernelGGL(k_kubo_post_sums, dim3(1), dim3(256), 0, st, nump, integrand, sigma);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }
@@ -595,8 +762,7 @@ int launch_greenwood_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, 
   return LQ_OK;
 }
 
-int launch_bastin_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, int n, double W, double Ec, int num_div,
-                          double *scratch, double *E, double *out) {
+int launch_bastin_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, int n, double W, double Ec, int num_div, double *scratch, double *E, double *out) {
   double *energies = scratch, *kern = scratch + num_div;
   const size_t lds = sizeof(double) * (size_t)M0;
   if (lds > 64 * 1024) {
@@ -605,7 +771,7 @@ int launch_bastin_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, int
   }
   hipLaunchKernelGGL(k_bastin_energies, dim3((num_div + 255) / 256), dim3(256), 0, st, num_div, energies);
   hipLaunchKernelGGL((k_grid2d<1>), dim3(num_div), dim3(256), lds, st, mu, M0, M1, energies, kern);
-  hipLaunchKernelGGL(k_bastin_finish, dim3(1), dim3(64), 0, st, num_div, n, W, Ec, energies, kern, E, out);
+  hipLaunchKernelGGL(k_bastin_finish, dim3(1), dim3(256), 0, st, num_div, n, W, Ec, energies, kern, E, out);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }
