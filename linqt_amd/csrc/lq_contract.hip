@@ -20,6 +20,7 @@
 // once per block, K is split into nsplit chunks, and the blocks of one chunk
 // run together on one XCD (block_chunk_tile).  A deterministic second pass
 // sums the chunks.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -713,46 +714,66 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(192))) void k_c
       }
 }
 
-__global__ void k_contract_reduce(const double2 *__restrict__ work, int nsplit, int M0, int M1,
-                                  double2 *__restrict__ out, int ldo, int accumulate) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)M0 * M1) return;
-  const int m = (int)(t / M1), nn = (int)(t % M1);
+// Sum of the nsplit partial tables at element t by the eight threads p = 0..7
+// that share it (32 elements to a block of 256): thread p adds the chunks p,
+// p + 8, ... in order, then the eight sums are added in order.  One thread per
+// element left small tables to a few wavefronts with a chain of up to 256 loads
+// each (100 x 100, 64 chunks: 19.5 us; 6 with eight threads).
+constexpr int kRedParts = 8, kRedElems = 32;
+__device__ __forceinline__ bool reduce_chunks(const double2 *__restrict__ work, int nsplit, long long total, long long t,
+                                              double2 &v) {
+  __shared__ double2 sh[kRedParts][kRedElems];
+  const int e = threadIdx.x % kRedElems, p = threadIdx.x / kRedElems;
   double sx = 0.0, sy = 0.0;
-  for (int c = 0; c < nsplit; ++c) {
-    const double2 w = work[((size_t)c * M0 + m) * M1 + nn];
-    sx += w.x;
-    sy += w.y;
+  if (t < total) {
+#pragma unroll 4
+    for (int c = p; c < nsplit; c += kRedParts) {
+      const double2 w = work[(size_t)c * total + t];
+      sx += w.x;
+      sy += w.y;
+    }
   }
+  sh[p][e] = make_double2(sx, sy);
+  __syncthreads();
+  if (p > 0 || t >= total) return false;
+  for (int u = 1; u < kRedParts; ++u) {
+    sx += sh[u][e].x;
+    sy += sh[u][e].y;
+  }
+  v = make_double2(sx, sy);
+  return true;
+}
+
+__global__ __launch_bounds__(256) void k_contract_reduce(const double2 *__restrict__ work, int nsplit, int M0, int M1,
+                                                         double2 *__restrict__ out, int ldo, int accumulate) {
+  const long long t = (long long)blockIdx.x * kRedElems + threadIdx.x % kRedElems;
+  double2 v;
+  if (!reduce_chunks(work, nsplit, (long long)M0 * M1, t, v)) return;
+  const int m = (int)(t / M1), nn = (int)(t % M1);
   double2 *o = out + (size_t)m * ldo + nn;
   if (accumulate) {
-    sx += o->x;
-    sy += o->y;
+    v.x += o->x;
+    v.y += o->y;
   }
-  *o = make_double2(sx, sy);
+  *o = v;
 }
 
 // The same sum for a table whose columns hold nout operators' blocks of bc
 // columns side by side: column o*bc + s goes to out_o[m*ldo + s].
-__global__ void k_contract_reduce_cols(const double2 *__restrict__ work, int nsplit, int M0, int M1, int bc,
-                                       double2 *__restrict__ out0, double2 *__restrict__ out1, int ldo,
-                                       int accumulate) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)M0 * M1) return;
+__global__ __launch_bounds__(256) void k_contract_reduce_cols(const double2 *__restrict__ work, int nsplit, int M0,
+                                                              int M1, int bc, double2 *__restrict__ out0,
+                                                              double2 *__restrict__ out1, int ldo, int accumulate) {
+  const long long t = (long long)blockIdx.x * kRedElems + threadIdx.x % kRedElems;
+  double2 v;
+  if (!reduce_chunks(work, nsplit, (long long)M0 * M1, t, v)) return;
   const int m = (int)(t / M1), nn = (int)(t % M1);
-  double sx = 0.0, sy = 0.0;
-  for (int c = 0; c < nsplit; ++c) {
-    const double2 w = work[((size_t)c * M0 + m) * M1 + nn];
-    sx += w.x;
-    sy += w.y;
-  }
   const int o = nn / bc, sc = nn % bc;
   double2 *o_ = (o == 0 ? out0 : out1) + (size_t)m * ldo + sc;
   if (accumulate) {
-    sx += o_->x;
-    sy += o_->y;
+    v.x += o_->x;
+    v.y += o_->y;
   }
-  *o_ = make_double2(sx, sy);
+  *o_ = v;
 }
 
 // Kernel choice for tables of at least 128 x 128: the three-multiplication
@@ -858,22 +879,39 @@ bool t128_fits(long long lda, long long ldb) {
   return lda <= lim && ldb <= lim;
 }
 
-// Split-K chunks.  The 128 x 128 kernel takes the chunks of the 128 x 64
-// kernels (its time does not depend on them: 46.2-46.3 ms at 16, 32 or 64
-// chunks for 512 x 512 x 2^21), so every three-product kernel sums the same
-// chunks in the same order and gives the same tables.
+// Split-K chunks: at least kMinChunk elements each, in whole XCD groups (multiples
+// of 8) where K allows.  The 64 x 64 kernel gets about eight blocks per CU.  The
+// others hold one 128 x 128 tile per CU (512 threads, 128 KB of LDS), so the
+// chunk count is the one that makes the rounds of 256 blocks shortest: rounds x
+// (chunk + start), plus the reduction of the partial tables, in units of one
+// element of a block (0.36 us at 70 TFLOP/s).  Every three-product kernel sums the
+// same chunks in the same order and gives the same tables.
+// Against chunks of at least 4096 elements and no look at the last round (us,
+// contraction + reduction): 100 x 100 x 8192 602 -> 36, 128 x 128 x 8192
+// 1438 -> 49, 300 x 300 x 54150 1484 -> 729, 512 x 512 x 8192 1450 -> 211; tables
+// with K in the millions keep their chunks.
+constexpr int kMinChunk = 64;
 int choose_nsplit(int M0, int M1, long long K) {
-  const int kind = contract_kind(M0, M1);
-  const int bm = kind == kWave ? 64 : kBT, bn = (kind == kLds3m || kind == kLds3m128) ? kBN3 : bm;
-  const int target = kind == kWave ? 2048 : 512;  // blocks in flight
-  const long long tiles = (long long)((M0 + bm - 1) / bm) * ((M1 + bn - 1) / bn);
-  long long ns = (target + tiles - 1) / tiles;
-  ns = ((ns + 7) / 8) * 8;  // whole XCD groups
-  if (ns > 256) ns = 256;
-  long long by_k = K / 4096;  // keep every chunk >= 4096 elements long
-  if (by_k < 1) by_k = 1;
-  if (ns > by_k) ns = by_k;
-  return (int)ns;
+  const long long by_k = std::max(1LL, K / kMinChunk);
+  if (contract_kind(M0, M1) == kWave) {
+    const long long tiles = (long long)((M0 + 63) / 64) * ((M1 + 63) / 64);
+    const long long ns = std::min<long long>(((2048 + tiles - 1) / tiles + 7) / 8 * 8, 512);
+    return (int)std::min(ns, by_k < 8 ? by_k : by_k / 8 * 8);
+  }
+  if (by_k < 8) return (int)by_k;
+  const long long tiles = (long long)((M0 + kBT - 1) / kBT) * ((M1 + kBT - 1) / kBT);
+  const double unit = 0.36e-6, bandwidth = 5e12;
+  long long best = 8;
+  double least = 1e300;
+  for (long long ns = 8; ns <= std::min<long long>(by_k, 256) && (ns == 8 || ns * tiles <= 1024); ns += 8) {
+    const double rounds = (double)((tiles * ns + 255) / 256), chunk = (double)((K + ns - 1) / ns + 15) / 16 * 16;
+    const double cost = rounds * (chunk + 16.0) + 16.0 * ns * M0 * (double)M1 / bandwidth / unit;
+    if (cost < 0.99 * least) {
+      least = cost;
+      best = ns;
+    }
+  }
+  return (int)best;
 }
 
 }  // namespace
@@ -948,7 +986,7 @@ int launch_contract_f64(hipStream_t st, const double2 *A, long long lda, int M0,
 int launch_contract_reduce(hipStream_t st, const double2 *work, int nsplit, int M0, int M1, double2 *out, int ldo,
                            int accumulate) {
   const long long total = (long long)M0 * M1;
-  hipLaunchKernelGGL(k_contract_reduce, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, work, nsplit, M0,
+  hipLaunchKernelGGL(k_contract_reduce, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st, work, nsplit, M0,
                      M1, out, ldo, accumulate);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
@@ -961,7 +999,7 @@ int launch_contract_reduce_cols(hipStream_t st, const double2 *work, int nsplit,
     return LQ_ERR_ARG;
   }
   const long long total = (long long)M0 * M1;
-  hipLaunchKernelGGL(k_contract_reduce_cols, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, work, nsplit,
+  hipLaunchKernelGGL(k_contract_reduce_cols, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st, work, nsplit,
                      M0, M1, bc, outs[0], M1 / bc > 1 ? outs[1] : outs[0], ldo, accumulate);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
