@@ -532,6 +532,7 @@ int build_dict_form(const lq_csr A, SellDev &d, const DevCsr &csr) {
   if (dict.empty()) dict.push_back(d2(0.0, 0.0));
   d.dstored = (long long)stored;
   d.dwmax = wmax;
+  d.duw = (long long)wmax * nslices * kSlice == (long long)stored ? wmax : -1;
   LQ_HIP_CHECK(hipMalloc(&d.dsptr, sizeof(int) * sptr.size()));
   LQ_HIP_CHECK(hipMalloc(&d.wcol, sizeof(unsigned) * (stored > 0 ? stored : 1)));
   LQ_HIP_CHECK(hipMalloc(&d.dict, sizeof(double2) * dict.size()));
@@ -606,6 +607,7 @@ int upload_sell(lq_csr A, const DevCsr *src = nullptr) {
   d.nslices = nslices;
   d.stored = (long long)stored;
   d.wmax = wmax;
+  d.uw = (long long)wmax * nslices * kSlice == (long long)stored ? wmax : -1;
   dict_schedule(d);
   // the CSR on the device for both fills (A's host arrays uploaded when no
   // device copy was handed in); on an error everything allocated here is freed
@@ -710,22 +712,27 @@ struct SpmvLoopGuard {
 // the separate applies they replace).
 int spmm(lq_ctx ctx, lq_csr A, double2 alpha, double2 beta, const VecSet *sets, int nsets, int dot_mode = kDotNone,
          const double2 *phi = nullptr, double2 *partial = nullptr, const FusedArgs *fused = nullptr,
-         double extra_bytes = 0.0) {
+         double extra_bytes = 0.0, int nd = 1) {
   int k = 0;
   for (int s = 0; s < nsets; ++s) k += sets[s].k;
   const double bytes = (double)spmv_bytes(A, k, sets[0].z != nullptr) + extra_bytes;
   if (ctx->spmv_loop) {
     ctx->loop_bytes += bytes;
     ctx->loop_launches++;
-    return launch_spmm(ctx->stream, A->dev, alpha, beta, sets, nsets, dot_mode, phi, partial, nullptr, fused);
+    return launch_spmm(ctx->stream, A->dev, alpha, beta, sets, nsets, dot_mode, phi, partial, nullptr, fused, nd);
   }
   hipEvent_t ev;
   LQ_TRY(time_begin(ctx, kCatSpmv, &ev));
-  LQ_TRY(launch_spmm(ctx->stream, A->dev, alpha, beta, sets, nsets, dot_mode, phi, partial, nullptr, fused));
+  LQ_TRY(launch_spmm(ctx->stream, A->dev, alpha, beta, sets, nsets, dot_mode, phi, partial, nullptr, fused, nd));
   return time_end(ctx, kCatSpmv, ev, bytes);
 }
 
 }  // namespace
+
+int dots_due(int m, int RS, int M, int next) {
+  const int p = m % RS;
+  return p % 3 == 2 || p == RS - 1 || m == M - 1 ? m - next + 1 : 0;
+}
 
 // A new operator around a host CSR already filled in (rowptr / col / val /
 // kind, rows sorted, columns ascending): uploads its device forms.
@@ -2066,9 +2073,12 @@ int lq_spectral_moments(lq_csr H, lq_csr OP, const double *phi, int R, int M, in
         if (ctx->graph_seen == key || (ctx->graph.exec && ctx->graph.key == key)) {
           LQ_TRY(recursion_chunk_graph(ctx, key, [&]() -> int {
             double2 *a = A, *b = B;
+            int next = 2;
             for (int m = 1; m + 1 < M; ++m) {
               VecSet s{b, a, a, gg};
-              LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, ring(m + 1)));
+              const int nd = dots_due(m + 1, RS, M, next);
+              LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, ring(m + 1), nullptr, 0.0, nd));
+              next += nd;
               std::swap(a, b);
             }
             return LQ_OK;
@@ -2085,6 +2095,7 @@ int lq_spectral_moments(lq_csr H, lq_csr OP, const double *phi, int R, int M, in
       {
         hipGraphExec_t chunk_graph = nullptr;
         const int graph_from = graphs_enabled() && !whole ? kPartRing : M;  // first moment a replay produces
+        int next = 2;  // first moment not taken
         for (int m = 1; m + 1 < M; ++m) {
           if ((m + 1) % RS == 0) LQ_TRY(flush(m + 1));
           if (m + 1 >= graph_from && (m + 1) % kPartRing == 0 && m + kPartRing < M) {
@@ -2092,9 +2103,12 @@ int lq_spectral_moments(lq_csr H, lq_csr OP, const double *phi, int R, int M, in
               GraphKey key{H->uid, H->version, A, B, phi_d, part0, n, gg, -kPartRing};  // < 0: a ring chunk
               LQ_TRY(recursion_chunk_graph(ctx, key, [&]() -> int {
                 double2 *a = A, *b = B;
+                int nq = 0;
                 for (int q = 0; q < kPartRing; ++q) {
                   VecSet s{b, a, a, gg};
-                  LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, part0 + (size_t)q * slot));
+                  const int nd = dots_due(q, kPartRing, kPartRing, nq);
+                  LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, part0 + (size_t)q * slot, nullptr, 0.0, nd));
+                  nq += nd;
                   std::swap(a, b);
                 }
                 return LQ_OK;
@@ -2104,11 +2118,14 @@ int lq_spectral_moments(lq_csr H, lq_csr OP, const double *phi, int R, int M, in
             ctx->loop_launches += kPartRing;
             ctx->loop_bytes += (double)kPartRing * spmv_bytes(H, gg, true);
             m += kPartRing - 1;  // an even count of steps: A and B end where they started
+            next = m + 2;
             continue;
           }
           // A <- 2 H~ B - A, then swap: after the step B holds T_{m+1}
           VecSet s{B, A, A, gg};
-          LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, ring(m + 1)));
+          const int nd = dots_due(m + 1, RS, M, next);
+          LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, phi_d, ring(m + 1), nullptr, 0.0, nd));
+          next += nd;
           std::swap(A, B);
         }
       }
@@ -2432,9 +2449,11 @@ int lq_time_correlations(lq_csr H, lq_csr OPL, lq_csr OPR, const double *phi, in
           VecSet s{A, nullptr, B, gg};
           LQ_TRY(spmm(ctx, H, one, zero, &s, 1, kDotPhi, pl, part + slot));
         }
-        for (int m = 1; m + 1 < M; ++m) {
+        for (int m = 1, next = 2; m + 1 < M; ++m) {
           VecSet s{B, A, A, gg};
-          LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, pl, part + (size_t)(m + 1) * slot));
+          const int nd = dots_due(m + 1, M, M, next);
+          LQ_TRY(spmm(ctx, H, two, mone, &s, 1, kDotPhi, pl, part + (size_t)(m + 1) * slot, nullptr, 0.0, nd));
+          next += nd;
           std::swap(A, B);
         }
         LQ_TRY(spmv_loop_end(ctx));

@@ -163,6 +163,8 @@ int admit(lq_batch b, Job &j) {
   d.dict = j.H->dev.dict;
   d.diag = j.H->dev.diag;
   d.ndict = j.H->dev.ndict;
+  d.uw = j.H->dev.uw;
+  d.duw = j.H->dev.duw;
   d.phi = (const double2 *)p;
   d.buf0 = (double2 *)(p + vec);
   d.buf1 = (double2 *)(p + 2 * vec);
@@ -237,7 +239,9 @@ int run_chunk(lq_batch b) {
       tab.clear();
       int grid = 0;
       double work = 0.0;
+      bool equal_slices = true;
       for (Job *j : kv.second) {
+        equal_slices = equal_slices && (j->d.ndict == 0 || j->d.duw >= 0);
         j->d.blk0 = grid;
         grid += j->nblk;
         tab.push_back(j->d);
@@ -258,7 +262,8 @@ int run_chunk(lq_batch b) {
       hipEvent_t ev;
       LQ_TRY(time_begin(ctx, kCatSpmv, &ev));
       for (int s = 0; s < L; ++s)
-        LQ_TRY(launch_spmm_batch(ctx->stream, kp, unroll, c.dev, (int)tab.size(), grid, b->tc, s));
+        LQ_TRY(launch_spmm_batch(ctx->stream, kp, unroll, c.dev, (int)tab.size(), grid, b->tc, s, L,
+                                 equal_slices));
       double bytes = 0.0;
       for (Job *j : kv.second) {
         const int active = std::min(L, j->d.t0 + j->d.steps - b->t);

@@ -78,6 +78,7 @@ struct SellDev {
   double2 *val = nullptr;// [stored]
   long long stored = 0;
   int wmax = 0;          // widest slice (entries per row)
+  int uw = -1;           // entries per row of every slice when all are as wide, else -1
   // dictionary form (ndict == 0: absent)
   int ndict = 0;
   int *dsptr = nullptr;      // [nslices+1]
@@ -86,6 +87,7 @@ struct SellDev {
   double2 *diag = nullptr;   // [n] (nullptr: zero diagonal)
   long long dstored = 0;
   int dwmax = 0;
+  int duw = -1;
   // schedule of the dictionary-form launches, fixed when the operator is
   // uploaded (dict_schedule): grid cap and prefetched row groups
   int gridcap = 0;
@@ -112,7 +114,13 @@ struct VecSet {
 // Dot-product fusion of the recursion kernel.
 enum DotMode {
   kDotNone = 0,
-  kDotPhi = 1,      // partial = sum_rows conj(phi[i][v]) * y[i][v]
+  // partial = sum_rows conj(phi[i][v]) * y[i][v], and for nd = 2, 3 moments also
+  // of the row's own x and z to the slots before partial (grid * KP values each);
+  // nd = 0: none.  Taking the moments of three steps together reads phi once
+  // instead of three times: 48.8 -> 44 us a step at N = 492723, 5 vectors, random
+  // hoppings (three vector streams and the operator, 200 MB), the same moments bit
+  // for bit.
+  kDotPhi = 1,
   kDotDoubling = 2  // partials = sum conj(x_i)x_i and sum conj(x_i) y_i (row's own x)
 };
 
@@ -141,6 +149,7 @@ struct FusedArgs {
   const double2 *vdiag[2] = {nullptr, nullptr};
   double2 *yv[2] = {nullptr, nullptr};
   int nt = 0;  // nonzero: yv stored and z loaded non-temporally (set by launch_spmm)
+  int nd = 1;  // kDotPhi: moments taken by this step (see DotMode; set by launch_spmm)
 };
 
 // One job of a batched recursion launch (device table entry).
@@ -154,6 +163,7 @@ struct BatchJobDev {
   const double2 *dict;
   const double2 *diag;
   int ndict;
+  int uw, duw;  // equal slice widths of the two forms (-1: not equal)
   const double2 *phi;  // [n][k] states
   double2 *buf0, *buf1;  // T_s ring
   double2 *partial;      // [chunk slot][nblk][k-width] dot partials
@@ -164,7 +174,11 @@ struct BatchJobDev {
 // Launchers (lq_spmv.hip).  Return LQ_OK or an error code.
 int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, const VecSet *sets,
                 int nsets, int dot_mode, const double2 *phi, double2 *partial, int *grid_used,
-                const FusedArgs *fused = nullptr);
+                const FusedArgs *fused = nullptr, int nd = 1);
+// Moments a direct recursion takes in the step that produces moment m, when the
+// moments below `next` are taken: three at a time, and what is left at the last
+// moment and at the end of a ring of RS partial slots (groups start anew there).
+int dots_due(int m, int RS, int M, int next);
 int spmm_dot_grid(int n, int kpad);  // number of blocks a dot-mode launch uses
 int launch_dot(hipStream_t st, int n, int k, const double2 *a, const double2 *b, double2 *partial,
                int *grid_used);
@@ -172,9 +186,10 @@ int launch_reduce_partials(hipStream_t st, const double2 *partial, int nslots, i
                            double2 *out);
 int launch_copy(hipStream_t st, double2 *dst, const double2 *src, size_t count);
 // Batched recursion (one width class kp, grid = sum of the jobs' nblk): step
-// slot of the chunk whose first launch index is *tc.
+// slot of the chunk of nslots steps whose first launch index is *tc.
+// equal_slices: every job in dictionary form has slices of one width.
 int launch_spmm_batch(hipStream_t st, int kp, int unroll, const BatchJobDev *jobs, int njobs, int grid,
-                      const int *tc, int slot);
+                      const int *tc, int slot, int nslots, bool equal_slices);
 int launch_batch_reduce(hipStream_t st, const BatchJobDev *jobs, int njobs, const int *tc, int nslots, int kp);
 int launch_set_int(hipStream_t st, int *p, int v);
 // dst[i*g + v] = src[(r0 + v)*n + i] (state-major device states -> [n][g]).

@@ -183,10 +183,12 @@ int lq_spectral_moments_noalloc(lq_csr H, lq_csr OP, const double *phi, int R, i
       VecSet s{T0, nullptr, T1, gg};
       LQ_TRY(launch_spmm(st, H->dev, one, zero, &s, 1, kDotPhi, phi_d, at(1), nullptr));
     }
-    for (int m = 1; m + 1 < M; ++m) {
+    for (int m = 1, next = 2; m + 1 < M; ++m) {
       if ((m + 1) % kNaRing == 0) LQ_TRY(flush(m + 1));
       VecSet s{T1, T0, T0, gg};
-      LQ_TRY(launch_spmm(st, H->dev, two, mone, &s, 1, kDotPhi, phi_d, at(m + 1), nullptr));
+      const int nd = dots_due(m + 1, kNaRing, M, next);
+      LQ_TRY(launch_spmm(st, H->dev, two, mone, &s, 1, kDotPhi, phi_d, at(m + 1), nullptr, nullptr, nd));
+      next += nd;
       std::swap(T0, T1);
     }
     LQ_TRY(flush(M));

@@ -30,14 +30,16 @@ struct SetArgs {
   int k[2];
 };
 
+// conj(a) * b; the same roundings wherever it is used (a moment's dot products
+// are equal bit for bit from every kernel that forms them)
 __device__ __forceinline__ double2 conj_mul(double2 a, double2 b) {
-  // conj(a) * b
-  return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
+  return make_double2(fma(a.x, b.x, a.y * b.y), fma(a.x, b.y, -(a.y * b.x)));
 }
 
+// Block sums of d[q], q < NDOT, to partial[q * qstride + slot + v], v < KP.
 template <int KP, int NDOT>
-__device__ __forceinline__ void block_reduce_store(double2 (&d)[2], double2 *partial, int slot) {
-  __shared__ double2 sh[2][256];
+__device__ __forceinline__ void block_reduce_store(const double2 *d, double2 (*sh)[256], double2 *partial,
+                                                   long long qstride, long long slot) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int q = 0; q < NDOT; ++q) sh[q][tid] = d[q];
@@ -55,8 +57,22 @@ __device__ __forceinline__ void block_reduce_store(double2 (&d)[2], double2 *par
   }
   if (tid < KP) {
 #pragma unroll
-    for (int q = 0; q < NDOT; ++q) partial[((size_t)slot * NDOT + q) * KP + tid] = sh[q][tid];
+    for (int q = 0; q < NDOT; ++q) partial[q * qstride + slot + tid] = sh[q][tid];
   }
+}
+
+// The nd (0..3) moments of a kDotPhi step: the step's own to partial, the ones
+// before it to the slots before, slot values apart.
+template <int KP>
+__device__ __forceinline__ void store_phi_dots(const double2 *d, int nd, double2 *partial, long long slot,
+                                               long long block) {
+  __shared__ double2 sh[3][256];
+  if (nd == 1)
+    block_reduce_store<KP, 1>(d, sh, partial, 0, block);
+  else if (nd == 2)
+    block_reduce_store<KP, 2>(d, sh, partial, -slot, block);
+  else if (nd == 3)
+    block_reduce_store<KP, 3>(d, sh, partial, -slot, block);
 }
 
 // MI355X has 8 XCDs and dispatches consecutive blocks round-robin over them.
@@ -73,7 +89,15 @@ __device__ __forceinline__ int xcd_group(int b, int q) { return (b % kXcds) * q 
 // value; dictionary: the packed word), column(w) gives the column and
 // value(w, a) the value (dictionary: looked up in the table).  diag() is the
 // separate diagonal of the dictionary form.
+// uw >= 0: every slice holds uw entries per row, so a slice's offset needs no
+// load (one memory round trip less before the words).
 struct PlainMat {
+  // z with the first entries (dictionary form, no PF): the fused Bastin step went
+  // from 86.6 to 73.7 us (N = 524288, 8 vectors, two operators), where z had been
+  // waited for on its own after the operators' stores.  The plain form, bound by
+  // its 20 bytes per entry, is 3 % slower that way and loads z last.
+  static constexpr bool kEarlyZ = false;
+  int uw;
   const int *__restrict__ sptr;
   const int *__restrict__ col;
   const double2 *__restrict__ val;
@@ -88,6 +112,8 @@ struct PlainMat {
 };
 
 struct DictMat {
+  static constexpr bool kEarlyZ = true;
+  int uw;
   const int *__restrict__ sptr;
   const unsigned *__restrict__ wcol;
   const double2 *dict;  // value table (LDS copy, or global in the batch kernel)
@@ -159,8 +185,9 @@ __device__ __forceinline__ void nt_store2(double2 *p, double2 a) {
   __builtin_nontemporal_store(v, (dvec2 *)p);
 }
 
-__device__ __forceinline__ void stage(double2 *dst, const double2 *__restrict__ src, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+// This thread's value of a table of n <= 256 (blocks of 256 threads).
+__device__ __forceinline__ double2 table_value(const double2 *__restrict__ src, int n) {
+  return (int)threadIdx.x < n ? src[threadIdx.x] : make_double2(0.0, 0.0);
 }
 
 // Rows of row groups g0, g0 + gstep, ... (RPB = 256 / KP rows each) of one
@@ -176,13 +203,14 @@ __device__ __forceinline__ void stage(double2 *dst, const double2 *__restrict__ 
 // The arithmetic is unchanged.
 constexpr int kPfGroups = 64;  // row groups per block covered by the staged offsets
 
-template <int KP, int DOT, int kUnroll, class Mat, int NV = 0, bool PF = false>
+// staged(): puts the value tables (and slice offsets) into LDS and meets the block's
+// barrier; operators with equal slices load their first words before it.  The
+// schedule PF over more than one slice per row group (KP < 4) is for those only.
+template <int KP, int DOT, int kUnroll, class Mat, int NV = 0, bool PF = false, class Staged>
 __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, double2 beta, const SetArgs &sa,
                                           int nrowgroups, const double2 *__restrict__ phi, int g0, int gstep,
-                                          double2 (&d)[2], const FusedArgs &fa = FusedArgs{},
-                                          const int2 *sgeo = nullptr) {
+                                          double2 (&d)[3], const FusedArgs &fa, const int2 *sgeo, Staged staged) {
   constexpr int RPB = 256 / KP;
-  static_assert(!PF || RPB <= 64, "staged offsets need row groups within one slice");
   const int tid = threadIdx.x;
   const int v = tid % KP;
   const int set = (v < sa.k[0]) ? 0 : 1;
@@ -205,7 +233,10 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
     }
   };
   auto geo = [&](int i, int gg, int &base_o, int &w_o) {
-    if (PF && i < kPfGroups) {
+    if (mat.uw >= 0) {
+      base_o = ((gg * RPB + tid / KP) >> 6) * mat.uw * kSlice;
+      w_o = mat.uw;
+    } else if (PF && i < kPfGroups) {
       const int2 q = sgeo[i];
       base_o = q.x;
       w_o = q.y;
@@ -222,14 +253,20 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
     if (gg < nrowgroups && rr < n && lane_on) geo(i, gg, bb, ww);
     fetch_chunk((size_t)bb + (rr & 63), ww);
   };
-  fetch(0, g0);
+  if (mat.uw >= 0) {
+    fetch(0, g0);
+    staged();
+  } else {
+    staged();
+    fetch(0, g0);
+  }
   int it = 0;
   for (int g = g0; g < nrowgroups; g += gstep, ++it) {
     const int row = g * RPB + tid / KP;
     if (row < n && lane_on) {
       const int r = row & 63;
       int base, w;
-      if (PF) {
+      if (PF || mat.uw >= 0) {
         geo(it, g, base, w);
       } else {
         const int s = row >> 6;
@@ -238,13 +275,12 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
       }
       const size_t p0 = (size_t)base + r;
       const size_t o = (size_t)row * kk + vv;
-      // The separate diagonal (dictionary form) and the row's own x: without
-      // PF loaded with the first entries; with PF loaded after the last chunk
-      // together with z (one round trip, and no registers held through the
-      // chunks).  Either way they enter the sums after the off-diagonal terms.
+      // The separate diagonal (dictionary form), the row's own x, z and phi:
+      // without PF loaded with the first entries; with PF loaded after the last
+      // chunk (one round trip, and no registers held through the chunks).  Either way they enter the sums after the off-diagonal terms.
       double2 dv = make_double2(0.0, 0.0), xo = make_double2(0.0, 0.0);
       double2 vdv[NV > 0 ? NV : 1];
-      double2 zv = make_double2(0.0, 0.0);
+      double2 zv = make_double2(0.0, 0.0), ph = make_double2(0.0, 0.0);
       auto own_loads = [&]() {
         bool vdg = false;
 #pragma unroll
@@ -256,7 +292,9 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
           }
         }
         if (mat.has_diag()) dv = mat.diag(row);
-        if (mat.has_diag() || vdg) xo = x[o];
+        if (mat.has_diag() || vdg || DOT == kDotDoubling || (DOT == kDotPhi && fa.nd > 1)) xo = x[o];
+        if (DOT == kDotPhi && fa.nd > 0) ph = phi[o];
+        if ((PF || Mat::kEarlyZ) && z) zv = fa.nt ? nt_load2(z + o) : z[o];
       };
       if (!PF) own_loads();
       double ar = 0.0, ai = 0.0;
@@ -326,10 +364,7 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
         }
       }
       if (PF && w <= 0) fetch(it + 1, g + gstep);
-      if (PF) {
-        own_loads();
-        if (z) zv = fa.nt ? nt_load2(z + o) : z[o];
-      }
+      if (PF) own_loads();
       if (vlane) {
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
@@ -351,19 +386,26 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
       }
       double2 res = make_double2(alpha.x * ar - alpha.y * ai, alpha.x * ai + alpha.y * ar);
       if (z) {
-        if (!PF) zv = fa.nt ? nt_load2(z + o) : z[o];
+        if (!PF && !Mat::kEarlyZ) zv = fa.nt ? nt_load2(z + o) : z[o];
         res.x += beta.x * zv.x - beta.y * zv.y;
         res.y += beta.x * zv.y + beta.y * zv.x;
       }
       y[o] = res;
       if (DOT == kDotPhi) {
-        const double2 t = conj_mul(phi[o], res);
+        // the step's own moment and the nd - 1 before it, whose vectors are at hand
+        const double2 t = conj_mul(ph, res);
         d[0].x += t.x;
         d[0].y += t.y;
+        if (fa.nd > 1) {
+          const double2 t1 = conj_mul(ph, xo), t2 = conj_mul(ph, zv);
+          d[1].x += t1.x;
+          d[1].y += t1.y;
+          d[2].x += t2.x;
+          d[2].y += t2.y;
+        }
       } else if (DOT == kDotDoubling) {
-        const double2 xi = x[o];
-        const double2 t0 = conj_mul(xi, xi);
-        const double2 t1 = conj_mul(xi, res);
+        const double2 t0 = conj_mul(xo, xo);
+        const double2 t1 = conj_mul(xo, res);
         d[0].x += t0.x;
         d[0].y += t0.y;
         d[1].x += t1.x;
@@ -382,47 +424,59 @@ struct MatArgs {
   const double2 *dict;
   const double2 *diag;
   int ndict;  // > 0: dictionary form
+  int uw;     // entries per row in every slice, -1: not the same
 };
 
 template <int KP, int DOT, int kUnroll, bool DICT, int NV = 0, bool PF = false>
 __global__ __launch_bounds__(256) void k_spmm(int n, MatArgs m, double2 alpha, double2 beta, SetArgs sa,
                                               int nrowgroups, const double2 *__restrict__ phi,
                                               double2 *__restrict__ partial, int q, FusedArgs fa) {
-  constexpr int NDOT = (DOT == kDotDoubling) ? 2 : 1;
-  double2 d[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+  double2 d[3] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
   // q > 0: one row group per block, XCD-remapped; q == 0: grid-stride loop
   const int g0 = q > 0 ? xcd_group(blockIdx.x, q) : blockIdx.x;
   const int gstep = q > 0 ? nrowgroups : gridDim.x;
   if (DICT) {
     __shared__ double2 sdict[256];
     __shared__ double2 svdict[NV > 0 ? NV : 1][NV > 0 ? 256 : 1];
-    stage(sdict, m.dict, m.ndict);
     __shared__ int2 sgeo[PF ? kPfGroups : 1];
-    if (PF) {
-      constexpr int RPB = 256 / KP;
-      for (int i = threadIdx.x; i < kPfGroups; i += blockDim.x) {
-        const int gg = g0 + i * gstep;
-        if (gg < nrowgroups) {
-          const int ss = (gg * RPB) >> 6;
-          const int b = m.sptr[ss];
-          sgeo[i] = make_int2(b, (m.sptr[ss + 1] - b) >> 6);
-        }
-      }
-    }
     FusedArgs fl = fa;
+    const double2 tv = table_value(m.dict, m.ndict);
+    double2 tvv[NV > 0 ? NV : 1];
 #pragma unroll
     for (int o = 0; o < NV; ++o) {
-      stage(svdict[o], fa.vdict[o], fa.nvdict[o]);
+      tvv[o] = table_value(fa.vdict[o], fa.nvdict[o]);
       fl.vdict[o] = svdict[o];
     }
-    __syncthreads();
-    const DictMat mat{m.sptr, m.wcol, sdict, m.diag};
-    spmm_body<KP, DOT, kUnroll, DictMat, NV, PF>(n, mat, alpha, beta, sa, nrowgroups, phi, g0, gstep, d, fl, sgeo);
+    auto staged = [&]() {
+      sdict[threadIdx.x] = tv;
+#pragma unroll
+      for (int o = 0; o < NV; ++o) svdict[o][threadIdx.x] = tvv[o];
+      if (PF && m.uw < 0) {
+        constexpr int RPB = 256 / KP;
+        for (int i = threadIdx.x; i < kPfGroups; i += blockDim.x) {
+          const int gg = g0 + i * gstep;
+          if (gg < nrowgroups) {
+            const int ss = (gg * RPB) >> 6;
+            const int b = m.sptr[ss];
+            sgeo[i] = make_int2(b, (m.sptr[ss + 1] - b) >> 6);
+          }
+        }
+      }
+      __syncthreads();
+    };
+    const DictMat mat{m.uw, m.sptr, m.wcol, sdict, m.diag};
+    spmm_body<KP, DOT, kUnroll, DictMat, NV, PF>(n, mat, alpha, beta, sa, nrowgroups, phi, g0, gstep, d, fl, sgeo,
+                                                 staged);
   } else {
-    const PlainMat mat{m.sptr, m.col, m.val};
-    spmm_body<KP, DOT, kUnroll>(n, mat, alpha, beta, sa, nrowgroups, phi, g0, gstep, d);
+    const PlainMat mat{m.uw, m.sptr, m.col, m.val};
+    spmm_body<KP, DOT, kUnroll, PlainMat>(n, mat, alpha, beta, sa, nrowgroups, phi, g0, gstep, d, fa, nullptr, [] {});
   }
-  if (DOT != kDotNone) block_reduce_store<KP, NDOT>(d, partial, blockIdx.x);
+  if constexpr (DOT == kDotDoubling) {
+    __shared__ double2 sh[2][256];
+    block_reduce_store<KP, 2>(d, sh, partial, KP, (long long)blockIdx.x * 2 * KP);
+  }
+  if constexpr (DOT == kDotPhi)
+    store_phi_dots<KP>(d, fa.nd, partial, (long long)gridDim.x * KP, (long long)blockIdx.x * KP);
 }
 
 // Batched recursion step over many independent jobs (one vector-width class):
@@ -434,7 +488,7 @@ __global__ __launch_bounds__(256) void k_spmm(int n, MatArgs m, double2 alpha, d
 //   s >= 1:  T_{s+1} = 2 H~ T_s - T_{s-1}     (in place over T_{s-1})
 template <int KP, int kUnroll, bool PF = false>
 __global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restrict__ jobs, int njobs,
-                                                    const int *__restrict__ tc, int slot, int ntz) {
+                                                    const int *__restrict__ tc, int slot, int nslots, int ntz) {
   int lo = 0, hi = njobs - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -457,34 +511,39 @@ __global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restric
   const double2 beta = s == 0 ? make_double2(0.0, 0.0) : make_double2(-1.0, 0.0);
   constexpr int RPB = 256 / KP;
   const int groups = (J.n + RPB - 1) / RPB;
-  double2 d[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+  double2 d[3] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+  FusedArgs bf;
+  bf.nt = ntz;
+  // moments are taken three at a time, the rest at the chunk's or the job's end
+  bf.nd = __builtin_amdgcn_readfirstlane(
+      slot % 3 == 2 || slot == nslots - 1 || s == J.steps - 1 ? min(slot % 3, s) + 1 : 0);
   if (J.ndict > 0) {
     __shared__ double2 sdict[256];
-    stage(sdict, J.dict, J.ndict);  // J is the same for the whole block
     __shared__ int2 sgeo[PF ? kPfGroups : 1];
-    if (PF) {
-      for (int i = threadIdx.x; i < kPfGroups; i += blockDim.x) {
-        const int gg = lb + i * J.nblk;
-        if (gg < groups) {
-          const int ss = (gg * RPB) >> 6;
-          const int b = J.dsptr[ss];
-          sgeo[i] = make_int2(b, (J.dsptr[ss + 1] - b) >> 6);
+    const double2 tv = table_value(J.dict, J.ndict);  // J is the same for the whole block
+    auto staged = [&]() {
+      sdict[threadIdx.x] = tv;
+      if (PF && J.duw < 0) {
+        for (int i = threadIdx.x; i < kPfGroups; i += blockDim.x) {
+          const int gg = lb + i * J.nblk;
+          if (gg < groups) {
+            const int ss = (gg * RPB) >> 6;
+            const int b = J.dsptr[ss];
+            sgeo[i] = make_int2(b, (J.dsptr[ss + 1] - b) >> 6);
+          }
         }
       }
-    }
-    __syncthreads();
-    const DictMat mat{J.dsptr, J.wcol, sdict, J.diag};
-    FusedArgs bf;
-    bf.nt = ntz;
-    spmm_body<KP, kDotPhi, kUnroll, DictMat, 0, PF>(J.n, mat, alpha, beta, sa, groups, J.phi, lb, J.nblk, d, bf,
-                                                    sgeo);
+      __syncthreads();
+    };
+    const DictMat mat{J.duw, J.dsptr, J.wcol, sdict, J.diag};
+    spmm_body<KP, kDotPhi, kUnroll, DictMat, 0, PF>(J.n, mat, alpha, beta, sa, groups, J.phi, lb, J.nblk, d, bf, sgeo,
+                                                    staged);
   } else {
-    const PlainMat mat{J.sptr, J.col, J.val};
-    FusedArgs bf;
-    bf.nt = ntz;
-    spmm_body<KP, kDotPhi, kUnroll>(J.n, mat, alpha, beta, sa, groups, J.phi, lb, J.nblk, d, bf);
+    const PlainMat mat{J.uw, J.sptr, J.col, J.val};
+    spmm_body<KP, kDotPhi, kUnroll, PlainMat>(J.n, mat, alpha, beta, sa, groups, J.phi, lb, J.nblk, d, bf, nullptr,
+                                              [] {});
   }
-  block_reduce_store<KP, 1>(d, J.partial + (size_t)slot * J.nblk * KP, lb);
+  store_phi_dots<KP>(d, bf.nd, J.partial + (size_t)slot * J.nblk * KP, (long long)J.nblk * KP, (long long)lb * KP);
 }
 
 // mom[(s + 1) * KP + v] = sum_b partial[slot][b][v] for every step s a job ran
@@ -561,7 +620,7 @@ __global__ __launch_bounds__(256) void k_dot(int n, int k, const double2 *__rest
   constexpr int RPB = 256 / KP;
   const int tid = threadIdx.x;
   const int v = tid % KP;
-  double2 d[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+  double2 d[1] = {make_double2(0.0, 0.0)};
   for (int g = blockIdx.x; g < nrowgroups; g += gridDim.x) {
     const int row = g * RPB + tid / KP;
     if (row < n && v < k) {
@@ -571,7 +630,8 @@ __global__ __launch_bounds__(256) void k_dot(int n, int k, const double2 *__rest
       d[0].y += t.y;
     }
   }
-  block_reduce_store<KP, 1>(d, partial, blockIdx.x);
+  __shared__ double2 sh[1][256];
+  block_reduce_store<KP, 1>(d, sh, partial, 0, (long long)blockIdx.x * KP);
 }
 
 // one block per slot: out[slot * width + w] = sum over b < grid of
@@ -632,8 +692,8 @@ void dict_schedule(SellDev &d) {
 namespace {
 
 MatArgs mat_args(const SellDev &A) {
-  if (use_dict(A)) return MatArgs{A.dsptr, nullptr, nullptr, A.wcol, A.dict, A.diag, A.ndict};
-  return MatArgs{A.sptr, A.col, A.val, nullptr, nullptr, nullptr, 0};
+  if (use_dict(A)) return MatArgs{A.dsptr, nullptr, nullptr, A.wcol, A.dict, A.diag, A.ndict, A.duw};
+  return MatArgs{A.sptr, A.col, A.val, nullptr, nullptr, nullptr, 0, A.uw};
 }
 
 // Prefetched schedule (dictionary form, up to 64 rows per group, no fused
@@ -681,8 +741,8 @@ void launch_k_spmm(hipStream_t st, int grid, int n, const MatArgs &m, double2 al
     }
     hipLaunchKernelGGL(kernel, dim3(gr), dim3(256), 0, st, n, m, alpha, beta, sa, groups, phi, partial, q, fa);
   };
-  if constexpr (DICT && NV == 0 && 256 / KP <= 64) {
-    if (q == 0 && pf) {
+  if constexpr (DICT && NV == 0) {
+    if (q == 0 && pf && (256 / KP <= 64 || m.uw >= 0)) {
       go(k_spmm<KP, DOT, U, DICT, NV, true>);
       return;
     }
@@ -788,7 +848,7 @@ int spmm_dot_grid(int n, int kpad) {
 }
 
 int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, const VecSet *sets, int nsets,
-                int dot_mode, const double2 *phi, double2 *partial, int *grid_used, const FusedArgs *fused) {
+                int dot_mode, const double2 *phi, double2 *partial, int *grid_used, const FusedArgs *fused, int nd) {
   // Fused steps store the operator products (read again only by the
   // contraction) and load T_{n-1} (read once) non-temporally, which leaves the
   // caches to the vectors the next step gathers: 5 % faster on the Bastin step.
@@ -799,6 +859,11 @@ int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, c
   FusedArgs fa = fused ? *fused : FusedArgs{};
   static const int nt = env_int("LQ_SPMM_NT", 1);
   fa.nt = fa.nv > 0 ? (nt > 0) : (nt >= 2);
+  fa.nd = nd;
+  if (dot_mode == kDotPhi && (nd < 0 || nd > 3 || (nd == 3 && !sets[0].z))) {
+    set_error("launch_spmm: %d moments of one step", nd);
+    return LQ_ERR_ARG;
+  }
   if (fa.nv < 0 || fa.nv > 2 || (fa.nv > 0 && (fa.set < 0 || fa.set >= nsets || !fa.vidx))) {
     set_error("launch_spmm: bad fused operator arguments");
     return LQ_ERR_ARG;
@@ -878,21 +943,21 @@ int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, c
 }
 
 int launch_spmm_batch(hipStream_t st, int kp, int unroll, const BatchJobDev *jobs, int njobs, int grid,
-                      const int *tc, int slot) {
+                      const int *tc, int slot, int nslots, bool equal_slices) {
   if (njobs <= 0 || grid <= 0) return LQ_OK;
   // T_{n-1} loaded non-temporally: the batch mix holds jobs whose vector
   // blocks exceed the MALL (0.8 % faster over the mix); LQ_SPMM_NT=0 turns it off
   static const int ntz = env_int("LQ_SPMM_NT", 1) >= 1 ? 1 : 0;
-#define LQ_BU(KPV, UV)                                                                                     \
-  if (kp == KPV && unroll == UV) {                                                                       \
-    if (256 / KPV <= 64 && spmm_pf())                                                                    \
-      hipLaunchKernelGGL((k_spmm_batch<KPV, UV, (256 / KPV <= 64)>), dim3(grid), dim3(256), 0, st, jobs,  \
-                         njobs, tc, slot, ntz);                                                          \
-    else                                                                                                 \
-      hipLaunchKernelGGL((k_spmm_batch<KPV, UV>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot,   \
-                         ntz);                                                                           \
-    LQ_HIP_CHECK(hipGetLastError());                                                                     \
-    return LQ_OK;                                                                                        \
+#define LQ_BU(KPV, UV)                                                                                        \
+  if (kp == KPV && unroll == UV) {                                                                          \
+    if ((256 / KPV <= 64 || equal_slices) && spmm_pf())                                                     \
+      hipLaunchKernelGGL((k_spmm_batch<KPV, UV, true>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot, \
+                         nslots, ntz);                                                                      \
+    else                                                                                                    \
+      hipLaunchKernelGGL((k_spmm_batch<KPV, UV>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot,      \
+                         nslots, ntz);                                                                      \
+    LQ_HIP_CHECK(hipGetLastError());                                                                        \
+    return LQ_OK;                                                                                           \
   }
 #define LQ_BK(KPV) LQ_BU(KPV, 4) LQ_BU(KPV, 8) LQ_BU(KPV, 12) LQ_BU(KPV, 16)
   LQ_BK(1)
