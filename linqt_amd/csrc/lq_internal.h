@@ -121,7 +121,8 @@ enum DotMode {
   // hoppings (three vector streams and the operator, 200 MB), the same moments bit
   // for bit.
   kDotPhi = 1,
-  kDotDoubling = 2  // partials = sum conj(x_i)x_i and sum conj(x_i) y_i (row's own x)
+  kDotDoubling = 2,  // partials = sum conj(x_i)x_i and sum conj(x_i) y_i (row's own x)
+  kDotSelf = 3       // partials = sum conj(y_i) y_i and sum conj(y_i) phi_i (one vector)
 };
 
 // Right operators applied inside the recursion step of H (at most 2; their

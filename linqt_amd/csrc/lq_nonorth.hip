@@ -10,15 +10,17 @@
 //   T0 = [OP] S^-1 phi,  T1 = S^-1 H T0,  T_{m+1} = 2 S^-1 H T_m - T_{m-1},
 //   mu_m += (2/R)(1/2 if m = 0) <phi|T_m>.
 //
-// Here every BiCGSTAB vector lives in HBM.  An iteration is two SpMVs with S
-// (the sliced-ELL kernel), three fused vector kernels (p/y, s/z, x/r) and
-// three reductions; the x/r update also produces |r|^2 and <r0|r> for the
-// next iteration, so the host reads three small results per iteration.
-// Reductions are two-level with a fixed order (per-block partials, then one
-// block), so a run is deterministic.
+// Here every BiCGSTAB vector and scalar lives in HBM.  An iteration is five
+// launches: p/y, v = S y with <r0|v>, s/z, t = S z with <t|t> and <t|s>, x/r with
+// |r|^2 and <r0|r>.  The kernels that need a dot product's value sum the partials
+// of the blocks before them, every block for itself, in one fixed order; the
+// stopping test is theirs too, and an iteration queued past it leaves the vectors
+// alone.  So the host queues as many iterations as the solve before took and only
+// then looks (one small copy), where a copy and a wait for each of three dot
+// products had taken most of an iteration's 100 us (N = 16380: 15.1 ms for 147
+// iterations in 49 solves).
 #include <algorithm>
 #include <cmath>
-#include <complex>
 #include <vector>
 
 #include "lq_internal.h"
@@ -120,43 +122,162 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_init(int n, const double2 *__
   block_store2(a, z, partial);
 }
 
-// p = r + beta (p - w v); y = dinv p
-__global__ __launch_bounds__(kNbThreads) void k_nb_p(int n, double2 beta, double2 w, const double2 *__restrict__ r,
-                                                      double2 *__restrict__ p, const double2 *__restrict__ v,
-                                                      const double2 *__restrict__ dinv, double2 *__restrict__ y) {
-  for (int i = blockIdx.x * kNbThreads + threadIdx.x; i < n; i += gridDim.x * kNbThreads) {
-    const double2 pi = cadd(r[i], cmul(beta, csub(p[i], cmul(w, v[i]))));
-    p[i] = pi;
-    y[i] = cmul(dinv[i], pi);
+// Scalars of a solve.  A kernel's block 0 writes the ones it computes; every
+// block of a kernel computes them for itself, and reads only what kernels before
+// it wrote (rho by parity of the iteration).
+enum NbState { kNbRunning = 0, kNbDone = 1, kNbRestart = 2 };
+struct NbScal {
+  double2 rho[2], alpha, w;
+  double rhs_sq, r0_sq, r_sq;
+  int state, it, i;
+};
+
+__device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
+  const double m = b.x * b.x + b.y * b.y;
+  return make_double2((a.x * b.x + a.y * b.y) / m, (a.y * b.x - a.x * b.y) / m);
+}
+
+// Every thread: (sum, sum) of nblk pairs (NV = 2) or single values of partials, in
+// one fixed order.
+template <int NV>
+__device__ __forceinline__ void sum_partials(const double2 *__restrict__ partial, int nblk, double2 &a, double2 &b) {
+  __shared__ double2 sh[2][kNbThreads];
+  const int t = threadIdx.x;
+  double2 u = make_double2(0.0, 0.0), v = u;
+  for (int q = t; q < nblk; q += kNbThreads) {
+    u = cadd(u, partial[NV * q]);
+    if (NV == 2) v = cadd(v, partial[NV * q + 1]);
+  }
+  sh[0][t] = u;
+  if (NV == 2) sh[1][t] = v;
+  __syncthreads();
+  for (int w = kNbThreads / 2; w > 0; w >>= 1) {
+    if (t < w) {
+      sh[0][t] = cadd(sh[0][t], sh[0][t + w]);
+      if (NV == 2) sh[1][t] = cadd(sh[1][t], sh[1][t + w]);
+    }
+    __syncthreads();
+  }
+  a = sh[0][0];
+  if (NV == 2) b = sh[1][0];
+}
+
+// Iteration i (the count-th that maxit bounds): the stopping test, rho and beta; then p = r + beta (p - w v), y =
+// dinv p.  partial: of |r|^2 and <r0|r> (first: of |b|^2).  resumed: after a
+// restart, rho and the test are settled.
+__global__ __launch_bounds__(kNbThreads) void k_nb_p(int n, int i, int count, int first, int resumed, double tol,
+                                                      int maxit, const double2 *__restrict__ partial, int nblk,
+                                                      NbScal *sc,
+                                                      const double2 *__restrict__ r, double2 *__restrict__ p,
+                                                      const double2 *__restrict__ v, const double2 *__restrict__ dinv,
+                                                      double2 *__restrict__ y) {
+  if (!first && !resumed && sc->state != kNbRunning) return;
+  const double2 one = make_double2(1.0, 0.0);
+  double2 rho, rho_old = first ? one : sc->rho[i & 1], alpha = first ? one : sc->alpha, w = first ? one : sc->w;
+  if (resumed) {
+    rho = sc->rho[(i + 1) & 1];
+  } else {
+    double2 rr, r0r;
+    sum_partials<2>(partial, nblk, rr, r0r);
+    if (first) r0r = make_double2(rr.x, 0.0);
+    const double rhs_sq = first ? rr.x : sc->rhs_sq, r0_sq = first ? rr.x : sc->r0_sq;
+    rho = r0r;
+    int state = kNbRunning;
+    if ((first && rhs_sq == 0.0) || !(rr.x > tol * tol * rhs_sq) || count >= maxit)
+      state = kNbDone;
+    else if (hypot(rho.x, rho.y) < 4.930380657631324e-32 * r0_sq)  // r too orthogonal to r0
+      state = kNbRestart;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc->state = state;
+      sc->r_sq = rr.x;
+      if (first) {
+        sc->rhs_sq = sc->r0_sq = rr.x;
+        sc->rho[i & 1] = sc->alpha = sc->w = one;
+      }
+      sc->it = count;
+      sc->i = i;
+      if (state == kNbRunning) sc->rho[(i + 1) & 1] = rho;
+    }
+    if (state != kNbRunning) return;
+  }
+  const double2 beta = cmul(cdiv(rho, rho_old), cdiv(alpha, w));
+  for (int e = blockIdx.x * kNbThreads + threadIdx.x; e < n; e += gridDim.x * kNbThreads) {
+    const double2 pi = cadd(r[e], cmul(beta, csub(p[e], cmul(w, v[e]))));
+    p[e] = pi;
+    y[e] = cmul(dinv[e], pi);
   }
 }
 
-// s = r - alpha v; z = dinv s
-__global__ __launch_bounds__(kNbThreads) void k_nb_s(int n, double2 alpha, const double2 *__restrict__ r,
+// alpha = rho / <r0|v> (partial); s = r - alpha v; z = dinv s
+__global__ __launch_bounds__(kNbThreads) void k_nb_s(int n, int i, const double2 *__restrict__ partial, int nblk,
+                                                      NbScal *sc, const double2 *__restrict__ r,
                                                       const double2 *__restrict__ v, const double2 *__restrict__ dinv,
                                                       double2 *__restrict__ s, double2 *__restrict__ z) {
-  for (int i = blockIdx.x * kNbThreads + threadIdx.x; i < n; i += gridDim.x * kNbThreads) {
-    const double2 si = csub(r[i], cmul(alpha, v[i]));
-    s[i] = si;
-    z[i] = cmul(dinv[i], si);
+  if (sc->state != kNbRunning) return;
+  double2 r0v, none;
+  sum_partials<1>(partial, nblk, r0v, none);
+  const double2 alpha = cdiv(sc->rho[(i + 1) & 1], r0v);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->alpha = alpha;
+  for (int e = blockIdx.x * kNbThreads + threadIdx.x; e < n; e += gridDim.x * kNbThreads) {
+    const double2 si = csub(r[e], cmul(alpha, v[e]));
+    s[e] = si;
+    z[e] = cmul(dinv[e], si);
   }
 }
 
-// x += alpha y + w z; r = s - w t; partials of |r|^2 and <r0|r>.
-__global__ __launch_bounds__(kNbThreads) void k_nb_xr(int n, double2 alpha, double2 w, double2 *__restrict__ x,
-                                                       const double2 *__restrict__ y, const double2 *__restrict__ z,
-                                                       const double2 *__restrict__ s, const double2 *__restrict__ t,
-                                                       double2 *__restrict__ r, const double2 *__restrict__ r0,
-                                                       double2 *__restrict__ partial) {
+// w = <t|s> / <t|t> (pin); x += alpha y + w z; r = s - w t; partials of |r|^2
+// and <r0|r>.
+__global__ __launch_bounds__(kNbThreads) void k_nb_xr(int n, const double2 *__restrict__ pin, int nblk, NbScal *sc,
+                                                       double2 *__restrict__ x, const double2 *__restrict__ y,
+                                                       const double2 *__restrict__ z, const double2 *__restrict__ s,
+                                                       const double2 *__restrict__ t, double2 *__restrict__ r,
+                                                       const double2 *__restrict__ r0, double2 *__restrict__ partial) {
+  if (sc->state != kNbRunning) return;
+  double2 tt, ts;
+  sum_partials<2>(pin, nblk, tt, ts);
+  const double2 alpha = sc->alpha;
+  const double2 w = tt.x > 0.0 ? make_double2(ts.x / tt.x, ts.y / tt.x) : make_double2(0.0, 0.0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->w = w;
   double2 a = make_double2(0.0, 0.0), b = make_double2(0.0, 0.0);
-  for (int i = blockIdx.x * kNbThreads + threadIdx.x; i < n; i += gridDim.x * kNbThreads) {
-    x[i] = cadd(x[i], cadd(cmul(alpha, y[i]), cmul(w, z[i])));
-    const double2 ri = csub(s[i], cmul(w, t[i]));
-    r[i] = ri;
+  for (int e = blockIdx.x * kNbThreads + threadIdx.x; e < n; e += gridDim.x * kNbThreads) {
+    x[e] = cadd(x[e], cadd(cmul(alpha, y[e]), cmul(w, z[e])));
+    const double2 ri = csub(s[e], cmul(w, t[e]));
+    r[e] = ri;
     a = cadd(a, cdot1(ri, ri));
-    b = cadd(b, cdot1(r0[i], ri));
+    b = cadd(b, cdot1(r0[e], ri));
   }
   block_store2(a, b, partial);
+}
+
+// After k_nb_restart of iteration i: r0_sq = rho = |r|^2 (partial), running again.
+__global__ __launch_bounds__(kNbThreads) void k_nb_resume(const double2 *__restrict__ partial, int nblk, int i,
+                                                           NbScal *sc) {
+  double2 rr, none;
+  sum_partials<2>(partial, nblk, rr, none);
+  if (threadIdx.x == 0) {
+    sc->r0_sq = rr.x;
+    sc->rho[(i + 1) & 1] = make_double2(rr.x, 0.0);
+    sc->state = kNbRunning;
+  }
+}
+
+// DiagonalPreconditioner from the sliced-ELL form: 1 / (the row's first diagonal
+// entry) when that is nonzero, else 1 (padding: own column, value 0).
+__global__ __launch_bounds__(kNbThreads) void k_nb_dinv(int n, const int *__restrict__ sptr,
+                                                         const int *__restrict__ col, const double2 *__restrict__ val,
+                                                         double2 *__restrict__ dinv) {
+  const int i = blockIdx.x * kNbThreads + threadIdx.x;
+  if (i >= n) return;
+  const int base = sptr[i / kSlice], w = (sptr[i / kSlice + 1] - base) / kSlice;
+  double2 d = make_double2(1.0, 0.0);
+  for (int j = 0; j < w; ++j) {
+    const size_t q = (size_t)base + (size_t)j * kSlice + i % kSlice;
+    if (col[q] != i) continue;
+    const double2 e = val[q];
+    if (e.x != 0.0 || e.y != 0.0) d = cdiv(make_double2(1.0, 0.0), e);
+    break;
+  }
+  dinv[i] = d;
 }
 
 // restart: r = r0 = b - t; partials of |r|^2
@@ -183,135 +304,100 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_cheb(int n, const double2 *__
 
 int nb_grid(int n) { return std::max(1, std::min(kNbBlocks, (n + kNbThreads - 1) / kNbThreads)); }
 
-struct NbBuf {
-  std::vector<void *> ptrs;
-  ~NbBuf() {
-    for (void *p : ptrs) (void)hipFree(p);
-  }
-  int alloc(size_t count, double2 **out) {
-    void *d = nullptr;
-    LQ_HIP_CHECK(hipMalloc(&d, sizeof(double2) * std::max<size_t>(count, 1)));
-    ptrs.push_back(d);
-    *out = (double2 *)d;
-    return LQ_OK;
-  }
-};
-
-// BiCGSTAB state on the device for systems with S (n rows).
+// BiCGSTAB state on the device for systems with S (n rows), in buffers of the
+// context that outlive the call (freed by lq_ctx_release).
 struct Bicg {
   lq_ctx ctx = nullptr;
   lq_csr S = nullptr;
-  int n = 0, grid = 1;
+  int n = 0, grid = 1, dots = 1;  // blocks of the vector kernels and of a product with dots
   double2 *r = nullptr, *r0 = nullptr, *p = nullptr, *v = nullptr, *y = nullptr, *z = nullptr, *s = nullptr,
-          *t = nullptr, *dinv = nullptr, *partial = nullptr, *res = nullptr;
+          *t = nullptr, *dinv = nullptr, *partial = nullptr, *dpart = nullptr, *res = nullptr;
+  NbScal *sc = nullptr, *host = nullptr;  // host: pinned
   long long iterations = 0;
+  int expect = 1;  // iterations the last solve took
 
-  int init(lq_ctx c, lq_csr S_, NbBuf &buf) {
+  int init(lq_ctx c, lq_csr S_) {
     ctx = c;
     S = S_;
     n = S->n;
     grid = nb_grid(n);
-    for (double2 **q : {&r, &r0, &p, &v, &y, &z, &s, &t, &dinv}) LQ_TRY(buf.alloc((size_t)n, q));
-    LQ_TRY(buf.alloc(2 * (size_t)kNbBlocks, &partial));
-    LQ_TRY(buf.alloc(2, &res));
-    // DiagonalPreconditioner: 1 / (first stored diagonal entry) when nonzero, else 1
-    std::vector<double2> h((size_t)n, make_double2(1.0, 0.0));
-    for (int i = 0; i < n; ++i)
-      for (int q = S->rowptr[i]; q < S->rowptr[i + 1]; ++q) {
-        if (S->kind[q] == 1) continue;  // mirrored entries are not part of the stored matrix
-        if (S->col[q] != i) continue;
-        const std::complex<double> d = S->val[q];
-        if (d != std::complex<double>(0.0)) {
-          const std::complex<double> inv = 1.0 / d;
-          h[i] = make_double2(inv.real(), inv.imag());
-        }
-        break;
-      }
-    LQ_HIP_CHECK(hipMemcpyAsync(dinv, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-    LQ_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    return LQ_OK;
-  }
-
-  // reduce the partials to res and read res[0..1] on the host
-  int reduce_read(std::complex<double> *a, std::complex<double> *b) {
-    hipLaunchKernelGGL(k_nb_final, dim3(1), dim3(kNbThreads), 0, ctx->stream, partial, grid, res, 0.0, nullptr);
+    dots = spmm_dot_grid(n, 1);
+    const size_t row = ((size_t)n + 15) / 16 * 16;
+    double2 *vec;
+    LQ_TRY(ctx_buf(ctx, "nb_vec", sizeof(double2) * 9 * row, (void **)&vec));
+    double2 **const all[9] = {&r, &r0, &p, &v, &y, &z, &s, &t, &dinv};
+    for (int q = 0; q < 9; ++q) *all[q] = vec + q * row;
+    LQ_TRY(ctx_buf(ctx, "nb_part", sizeof(double2) * (2 * (size_t)kNbBlocks + 2 * (size_t)dots + 2), (void **)&partial));
+    dpart = partial + 2 * (size_t)kNbBlocks;
+    res = dpart + 2 * (size_t)dots;
+    LQ_TRY(ctx_buf(ctx, "nb_scal", sizeof(NbScal), (void **)&sc));
+    LQ_TRY(ctx_pinned(ctx, sizeof(NbScal), (void **)&host));
+    hipLaunchKernelGGL(k_nb_dinv, dim3((n + kNbThreads - 1) / kNbThreads), dim3(kNbThreads), 0, ctx->stream, n,
+                       S->dev.sptr, S->dev.col, S->dev.val, dinv);
     LQ_HIP_CHECK(hipGetLastError());
-    double2 h[2];
-    LQ_HIP_CHECK(hipMemcpyAsync(h, res, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-    LQ_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    if (a) *a = {h[0].x, h[0].y};
-    if (b) *b = {h[1].x, h[1].y};
     return LQ_OK;
   }
 
-  int apply_S(const double2 *in, double2 *out) {
-    return lq_spmv(S, 1.0, 0.0, (const double *)in, 0.0, 0.0, (double *)out, 1);
+  int apply_S(const double2 *in, double2 *out, int dot_mode, const double2 *phi) {
+    VecSet set{in, nullptr, out, 1};
+    hipEvent_t ev;
+    LQ_TRY(time_begin(ctx, kCatSpmv, &ev));
+    LQ_TRY(launch_spmm(ctx->stream, S->dev, make_double2(1.0, 0.0), make_double2(0.0, 0.0), &set, 1, dot_mode, phi,
+                       dot_mode == kDotNone ? nullptr : dpart, nullptr));
+    return time_end(ctx, kCatSpmv, ev, 20.0 * (double)S->col.size() + 4.0 * (n + 1) + 32.0 * n);
   }
 
   // x = S^-1 b (Eigen's BiCGSTAB); b and x are distinct device vectors of n.
   int solve(const double2 *b, double2 *x, double tol, int maxit, int *iters, double *error) {
-    typedef std::complex<double> C;
     const dim3 g(grid), blk(kNbThreads);
-    hipLaunchKernelGGL(k_nb_init, g, blk, 0, ctx->stream, n, b, r, r0, x, p, v, partial);
+    const hipStream_t st = ctx->stream;
+    hipLaunchKernelGGL(k_nb_init, g, blk, 0, st, n, b, r, r0, x, p, v, partial);
     LQ_HIP_CHECK(hipGetLastError());
-    C rhs;
-    LQ_TRY(reduce_read(&rhs, nullptr));
-    const double rhs_sq = rhs.real();
-    int it = 0;
-    if (rhs_sq == 0.0) {
-      if (iters) *iters = 0;
-      if (error) *error = 0.0;
+    // i numbers the iterations queued (rho is stored by its parity); the count that
+    // maxit bounds starts anew at the first restart, as the sources' does
+    int i = 0, base = 0, restarts = 0, queue = expect + 1;
+    bool first = true, resumed = false;
+    auto rest = [&]() -> int {  // iteration i after its k_nb_p
+      LQ_TRY(apply_S(y, v, kDotPhi, r0));
+      hipLaunchKernelGGL(k_nb_s, g, blk, 0, st, n, i, dpart, dots, sc, r, v, dinv, s, z);
+      LQ_TRY(apply_S(z, t, kDotSelf, s));
+      hipLaunchKernelGGL(k_nb_xr, g, blk, 0, st, n, dpart, dots, sc, x, y, z, s, t, r, r0, partial);
+      LQ_HIP_CHECK(hipGetLastError());
       return LQ_OK;
-    }
-    double r0_sq = rhs_sq, r_sq = rhs_sq;
-    C r0r = rhs_sq, rho = 1.0, alpha = 1.0, w = 1.0;
-    const double tol2 = tol * tol * rhs_sq;
-    const double eps = 2.220446049250313e-16, eps2 = eps * eps;
-    int restarts = 0;
-    while (r_sq > tol2 && it < maxit) {
-      const C rho_old = rho;
-      rho = r0r;
-      if (std::abs(rho) < eps2 * r0_sq) {  // r too orthogonal to r0: restart from the current x
-        LQ_TRY(apply_S(x, t));
-        hipLaunchKernelGGL(k_nb_restart, g, blk, 0, ctx->stream, n, b, t, r, r0, partial);
+    };
+    for (;;) {
+      // `queue` stopping tests with the iterations between them, then a look
+      for (int q = 0;; ++q) {
+        hipLaunchKernelGGL(k_nb_p, g, blk, 0, st, n, i, i - base, first ? 1 : 0, resumed ? 1 : 0, tol, maxit, partial,
+                           grid, sc, r, p, v, dinv, y);
         LQ_HIP_CHECK(hipGetLastError());
-        C rr;
-        LQ_TRY(reduce_read(&rr, nullptr));
-        r0_sq = rr.real();
-        rho = r0_sq;
-        if (restarts++ == 0) it = 0;
+        first = resumed = false;
+        if (q + 1 >= queue) break;
+        LQ_TRY(rest());
+        ++i;
       }
-      const C beta = (rho / rho_old) * (alpha / w);
-      hipLaunchKernelGGL(k_nb_p, g, blk, 0, ctx->stream, n, make_double2(beta.real(), beta.imag()),
-                         make_double2(w.real(), w.imag()), r, p, v, dinv, y);
-      LQ_HIP_CHECK(hipGetLastError());
-      LQ_TRY(apply_S(y, v));
-      hipLaunchKernelGGL(k_nb_dot2, g, blk, 0, ctx->stream, n, r0, v, nullptr, nullptr, partial);
-      LQ_HIP_CHECK(hipGetLastError());
-      C r0v;
-      LQ_TRY(reduce_read(&r0v, nullptr));
-      alpha = rho / r0v;
-      hipLaunchKernelGGL(k_nb_s, g, blk, 0, ctx->stream, n, make_double2(alpha.real(), alpha.imag()), r, v, dinv, s,
-                         z);
-      LQ_HIP_CHECK(hipGetLastError());
-      LQ_TRY(apply_S(z, t));
-      hipLaunchKernelGGL(k_nb_dot2, g, blk, 0, ctx->stream, n, t, t, t, s, partial);
-      LQ_HIP_CHECK(hipGetLastError());
-      C tt, ts;
-      LQ_TRY(reduce_read(&tt, &ts));
-      const double tmp = tt.real();
-      w = tmp > 0.0 ? ts / tmp : C(0.0);
-      hipLaunchKernelGGL(k_nb_xr, g, blk, 0, ctx->stream, n, make_double2(alpha.real(), alpha.imag()),
-                         make_double2(w.real(), w.imag()), x, y, z, s, t, r, r0, partial);
-      LQ_HIP_CHECK(hipGetLastError());
-      C rr;
-      LQ_TRY(reduce_read(&rr, &r0r));
-      r_sq = rr.real();
-      ++it;
+      LQ_HIP_CHECK(hipMemcpyAsync(host, sc, sizeof(NbScal), hipMemcpyDeviceToHost, st));
+      LQ_HIP_CHECK(hipStreamSynchronize(st));
+      if (host->state == kNbDone) break;
+      if (host->state == kNbRestart) {  // from the current x, within iteration host->i
+        LQ_TRY(apply_S(x, t, kDotNone, nullptr));
+        i = host->i;
+        if (restarts++ == 0) base = i;
+        hipLaunchKernelGGL(k_nb_restart, g, blk, 0, st, n, b, t, r, r0, partial);
+        hipLaunchKernelGGL(k_nb_resume, dim3(1), blk, 0, st, partial, grid, i, sc);
+        LQ_HIP_CHECK(hipGetLastError());
+        resumed = true;
+        queue = 2;
+      } else {  // the last test went on
+        LQ_TRY(rest());
+        ++i;
+        queue = 1 + std::min(8, (i - base) / 4);
+      }
     }
-    iterations += it;
-    if (iters) *iters = it;
-    if (error) *error = std::sqrt(r_sq / rhs_sq);
+    iterations += host->it;
+    expect = host->it;
+    if (iters) *iters = host->it;
+    if (error) *error = host->rhs_sq == 0.0 ? 0.0 : std::sqrt(host->r_sq / host->rhs_sq);
     return LQ_OK;
   }
 };
@@ -337,9 +423,8 @@ extern "C" int lq_overlap_solve(lq_csr S, const double *b, double *x, double tol
   }
   lq_ctx ctx = S->ctx;
   DeviceGuard g(ctx->device);
-  NbBuf buf;
   Bicg bc;
-  LQ_TRY(bc.init(ctx, S, buf));
+  LQ_TRY(bc.init(ctx, S));
   return bc.solve((const double2 *)b, (double2 *)x, tol > 0 ? tol : 1e-4, maxit > 0 ? maxit : 2000, iterations,
                   error);
 } LQ_ABI_CATCH
@@ -361,12 +446,13 @@ extern "C" int lq_spectral_moments_nonorth(lq_csr H, lq_csr OP, lq_csr S, const 
   maxit = maxit > 0 ? maxit : 2000;
   lq_ctx ctx = H->ctx;
   DeviceGuard g(ctx->device);
-  NbBuf buf;
   Bicg bc;
-  LQ_TRY(bc.init(ctx, S, buf));
-  double2 *c0, *c1, *tmp, *tmp2, *ph, *dmu;
-  for (double2 **q : {&c0, &c1, &tmp, &tmp2, &ph}) LQ_TRY(buf.alloc((size_t)n, q));
-  LQ_TRY(buf.alloc((size_t)M, &dmu));
+  LQ_TRY(bc.init(ctx, S));
+  const size_t row = ((size_t)n + 15) / 16 * 16;
+  double2 *vec, *dmu;
+  LQ_TRY(ctx_buf(ctx, "nb_cheb", sizeof(double2) * 5 * row, (void **)&vec));
+  LQ_TRY(ctx_buf(ctx, "nb_mu", sizeof(double2) * (size_t)M, (void **)&dmu));
+  double2 *c0 = vec, *c1 = vec + row, *tmp = vec + 2 * row, *tmp2 = vec + 3 * row, *ph = vec + 4 * row;
   LQ_HIP_CHECK(hipMemcpyAsync(dmu, mu, sizeof(double2) * (size_t)M, hipMemcpyHostToDevice, ctx->stream));
   const dim3 gr(bc.grid), blk(kNbThreads);
   for (int r = 0; r < R; ++r) {

@@ -293,7 +293,7 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
         }
         if (mat.has_diag()) dv = mat.diag(row);
         if (mat.has_diag() || vdg || DOT == kDotDoubling || (DOT == kDotPhi && fa.nd > 1)) xo = x[o];
-        if (DOT == kDotPhi && fa.nd > 0) ph = phi[o];
+        if (DOT == kDotSelf || (DOT == kDotPhi && fa.nd > 0)) ph = phi[o];
         if ((PF || Mat::kEarlyZ) && z) zv = fa.nt ? nt_load2(z + o) : z[o];
       };
       if (!PF) own_loads();
@@ -410,6 +410,12 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
         d[0].y += t0.y;
         d[1].x += t1.x;
         d[1].y += t1.y;
+      } else if (DOT == kDotSelf) {
+        const double2 t0 = conj_mul(res, res), t1 = conj_mul(res, ph);
+        d[0].x += t0.x;
+        d[0].y += t0.y;
+        d[1].x += t1.x;
+        d[1].y += t1.y;
       }
     }
   }
@@ -471,7 +477,7 @@ __global__ __launch_bounds__(256) void k_spmm(int n, MatArgs m, double2 alpha, d
     const PlainMat mat{m.uw, m.sptr, m.col, m.val};
     spmm_body<KP, DOT, kUnroll, PlainMat>(n, mat, alpha, beta, sa, nrowgroups, phi, g0, gstep, d, fa, nullptr, [] {});
   }
-  if constexpr (DOT == kDotDoubling) {
+  if constexpr (DOT == kDotDoubling || DOT == kDotSelf) {
     __shared__ double2 sh[2][256];
     block_reduce_store<KP, 2>(d, sh, partial, KP, (long long)blockIdx.x * 2 * KP);
   }
@@ -795,6 +801,12 @@ int launch_spmm_kpu(hipStream_t st, const SellDev &A, double2 alpha, double2 bet
     case kDotDoubling:
       launch_k_spmm<KP, kDotDoubling, U, DICT, 0>(st, grid, A.n, m, alpha, beta, sa, groups, phi, partial, 0, fa, A.pf);
       break;
+    case kDotSelf:
+      if constexpr (KP == 1) {
+        launch_k_spmm<KP, kDotSelf, U, DICT, 0>(st, grid, A.n, m, alpha, beta, sa, groups, phi, partial, 0, fa, A.pf);
+        break;
+      }
+      [[fallthrough]];
     default:
       set_error("launch_spmm: bad dot mode %d", dot_mode);
       return LQ_ERR_ARG;
