@@ -122,7 +122,8 @@ enum DotMode {
   // for bit.
   kDotPhi = 1,
   kDotDoubling = 2,  // partials = sum conj(x_i)x_i and sum conj(x_i) y_i (row's own x)
-  kDotSelf = 3       // partials = sum conj(y_i) y_i and sum conj(y_i) phi_i (one vector)
+  kDotSelf = 3,      // partials = sum conj(y_i) y_i and sum conj(y_i) phi_i (one vector)
+  kDotAcc = 4        // no dots: acc (+)= ca[0] z + ca[1] x + ca[2] y per set (see FusedArgs)
 };
 
 // Right operators applied inside the recursion step of H (at most 2; their
@@ -151,6 +152,11 @@ struct FusedArgs {
   double2 *yv[2] = {nullptr, nullptr};
   int nt = 0;  // nonzero: yv stored and z loaded non-temporally (set by launch_spmm)
   int nd = 1;  // kDotPhi: moments taken by this step (see DotMode; set by launch_spmm)
+  // kDotAcc: the last na of the terms ca[0] z, ca[1] x, ca[2] y (row's own) are
+  // added to acc[set] in that order, which is overwritten when acc_new
+  int na = 0, acc_new = 0;
+  double2 ca[3] = {};
+  double2 *acc[2] = {nullptr, nullptr};
 };
 
 // One job of a batched recursion launch (device table entry).

@@ -292,8 +292,11 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
           }
         }
         if (mat.has_diag()) dv = mat.diag(row);
-        if (mat.has_diag() || vdg || DOT == kDotDoubling || (DOT == kDotPhi && fa.nd > 1)) xo = x[o];
+        if (mat.has_diag() || vdg || DOT == kDotDoubling || (DOT == kDotPhi && fa.nd > 1) ||
+            (DOT == kDotAcc && fa.na > 1))
+          xo = x[o];
         if (DOT == kDotSelf || (DOT == kDotPhi && fa.nd > 0)) ph = phi[o];
+        if (DOT == kDotAcc && fa.na > 0 && !fa.acc_new) ph = (set ? fa.acc[1] : fa.acc[0])[o];
         if ((PF || Mat::kEarlyZ) && z) zv = fa.nt ? nt_load2(z + o) : z[o];
       };
       if (!PF) own_loads();
@@ -410,6 +413,17 @@ __device__ __forceinline__ void spmm_body(int n, const Mat &mat, double2 alpha, 
         d[0].y += t0.y;
         d[1].x += t1.x;
         d[1].y += t1.y;
+      } else if (DOT == kDotAcc) {
+        if (fa.na > 0) {
+          auto add = [&](double2 c, double2 t) {
+            ph.x += fma(c.x, t.x, -(c.y * t.y));
+            ph.y += fma(c.x, t.y, c.y * t.x);
+          };
+          if (fa.na > 2) add(fa.ca[0], zv);
+          if (fa.na > 1) add(fa.ca[1], xo);
+          add(fa.ca[2], res);
+          (set ? fa.acc[1] : fa.acc[0])[o] = ph;
+        }
       } else if (DOT == kDotSelf) {
         const double2 t0 = conj_mul(res, res), t1 = conj_mul(res, ph);
         d[0].x += t0.x;
@@ -762,7 +776,7 @@ int launch_spmm_kpu(hipStream_t st, const SellDev &A, double2 alpha, double2 bet
   constexpr int RPB = 256 / KP;
   const int groups = (A.n + RPB - 1) / RPB;
   int grid = groups, q = 0;
-  if (dot_mode != kDotNone) {
+  if (dot_mode != kDotNone && dot_mode != kDotAcc) {
     grid = groups < kDotGridCap ? groups : kDotGridCap;
   } else if (DICT) {
     grid = A.gridcap > 0 ? (groups < A.gridcap ? groups : A.gridcap) : -1;  // -1: resident set
@@ -800,6 +814,9 @@ int launch_spmm_kpu(hipStream_t st, const SellDev &A, double2 alpha, double2 bet
       break;
     case kDotDoubling:
       launch_k_spmm<KP, kDotDoubling, U, DICT, 0>(st, grid, A.n, m, alpha, beta, sa, groups, phi, partial, 0, fa, A.pf);
+      break;
+    case kDotAcc:
+      launch_k_spmm<KP, kDotAcc, U, DICT, 0>(st, grid, A.n, m, alpha, beta, sa, groups, phi, partial, q, fa, A.pf);
       break;
     case kDotSelf:
       if constexpr (KP == 1) {
@@ -880,6 +897,15 @@ int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, c
     set_error("launch_spmm: bad fused operator arguments");
     return LQ_ERR_ARG;
   }
+  if (dot_mode == kDotAcc && fa.na > 0) {
+    bool ok = fused && fa.nv == 0 && fa.na <= 3;
+    for (int s = 0; ok && s < nsets; ++s) ok = fa.acc[s] && (fa.na < 3 || sets[s].z);
+    if (!ok) {
+      set_error("launch_spmm: bad accumulation arguments");
+      return LQ_ERR_ARG;
+    }
+    if (nsets == 1) fa.acc[1] = fa.acc[0];
+  }
   if (nsets < 1 || nsets > 2) {
     set_error("launch_spmm: nsets must be 1 or 2");
     return LQ_ERR_ARG;
@@ -903,7 +929,7 @@ int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, c
     sa.y[1] = sa.y[0];
     sa.k[1] = 0;
   }
-  if (dot_mode != kDotNone && nsets != 1) {
+  if (dot_mode != kDotNone && dot_mode != kDotAcc && nsets != 1) {
     set_error("launch_spmm: dot fusion needs a single vector set");
     return LQ_ERR_ARG;
   }
