@@ -3,9 +3,9 @@
 // Each job is chebyshev::SpectralMoments with OP = identity
 // (src/chebyshev_solver.cpp:176-200) for its own H~, states and M.  Instead of
 // one launch per step per job, a chunk of `chunk` recursion steps is issued
-// as one grouped launch per step per vector-width class (k_spmm_batch), so
-// small lattices that cannot fill the GPU alone share it, and the launch count
-// no longer grows with the number of jobs.
+// as one grouped launch per step (k_spmm_batch; a second one for jobs of 1 or 2
+// vectors with unequal slices), so small lattices that cannot fill the GPU alone share
+// it, and the launch count does not grow with the number of jobs.
 //
 // * Admission: jobs queue in submission order and are admitted first-fit at
 //   chunk boundaries while their device footprint (states, two recursion
@@ -17,7 +17,7 @@
 //   reduction order depend on the job alone, so its moments are bitwise the
 //   same alone, in any mix, and through lq_spectral_moments (R <= 64).
 // * Tuning: the unroll width of the gathers does not change the arithmetic;
-//   the first chunks of each width class try 4/8/12/16 and keep the fastest
+//   the first chunks of each of the two kernels try 4/8/12/16 and keep the fastest
 //   per row-step (LQ_BATCH_UNROLL fixes it).
 #include <algorithm>
 #include <chrono>
@@ -172,6 +172,7 @@ int admit(lq_batch b, Job &j) {
   d.mom = (double2 *)(p + 3 * vec + (size_t)b->chunk * j.nblk * j.kp * sizeof(double2));
   d.n = j.n;
   d.k = j.R;
+  d.kp = j.kp;
   d.t0 = b->t;
   d.steps = j.M - 1;
   d.nblk = j.nblk;
@@ -205,6 +206,10 @@ int harvest(lq_batch b, Job &j) {
   return LQ_OK;
 }
 
+double step_bytes(const Job &j) {
+  return 20.0 * j.H->col.size() + 4.0 * (j.n + 1) + 48.0 * j.R * (double)j.n;
+}
+
 int run_chunk(lq_batch b) {
   lq_ctx ctx = b->ctx;
   // admission, first fit in submission order
@@ -217,7 +222,13 @@ int run_chunk(lq_batch b) {
       ++q;
     }
   }
-  // running jobs by width class, in id order
+  // Running jobs by kernel (prefetched schedule or not), then by vector width: one
+  // launch steps them all.  A launch for each width left the chip half empty and
+  // paid 4 to 5 us a launch: 12 jobs up to N = 180000, widths 1 to 8: 15.5 ->
+  // 11.2 ms; 16 jobs up to N = 250000: 17.9 -> 14.9; 4 jobs up to 30000: 3.9 ->
+  // 1.8.  Sharing a launch only up to 150 or 200 MB swept in a step kept less
+  // (12.8 and 15.9 ms).
+  std::map<int, std::vector<Job *>> width;
   std::map<int, std::vector<Job *>> by;
   int L = 0;
   for (auto &kv : b->jobs) {
@@ -225,23 +236,24 @@ int run_chunk(lq_batch b) {
     if (j.state != 1) continue;
     const int left = j.d.t0 + j.d.steps - b->t;
     if (left > 0) {
-      by[j.kp].push_back(&j);
+      width[j.kp].push_back(&j);
       L = std::max(L, left);
     }
   }
+  for (auto &kv : width)
+    for (Job *j : kv.second)
+      by[spmm_batch_pf(j->kp, j->d.ndict == 0 || j->d.duw >= 0)].push_back(j);
   L = std::min(L, b->chunk);
   if (L > 0) {
     LQ_TRY(launch_set_int(ctx->stream, b->tc, b->t));
     for (auto &kv : by) {
-      const int kp = kv.first;
-      auto &c = b->cls[kp];
+      const bool pf = kv.first;
+      auto &c = b->cls[kv.first];
       std::vector<BatchJobDev> &tab = c.host;
       tab.clear();
       int grid = 0;
       double work = 0.0;
-      bool equal_slices = true;
       for (Job *j : kv.second) {
-        equal_slices = equal_slices && (j->d.ndict == 0 || j->d.duw >= 0);
         j->d.blk0 = grid;
         grid += j->nblk;
         tab.push_back(j->d);
@@ -255,19 +267,18 @@ int run_chunk(lq_batch b) {
       }
       LQ_HIP_CHECK(hipMemcpyAsync(c.dev, tab.data(), tab.size() * sizeof(BatchJobDev), hipMemcpyHostToDevice,
                                   ctx->stream));
-      Tune &tu = b->tune[kp];
+      Tune &tu = b->tune[kv.first];
       int unroll = b->fixed_unroll ? b->fixed_unroll : (tu.best ? tu.best : kUnrolls[tu.next]);
       const bool timing = !b->fixed_unroll && !tu.best;
       if (timing) LQ_HIP_CHECK(hipEventRecord(b->ev0, ctx->stream));
       hipEvent_t ev;
       LQ_TRY(time_begin(ctx, kCatSpmv, &ev));
       for (int s = 0; s < L; ++s)
-        LQ_TRY(launch_spmm_batch(ctx->stream, kp, unroll, c.dev, (int)tab.size(), grid, b->tc, s, L,
-                                 equal_slices));
+        LQ_TRY(launch_spmm_batch(ctx->stream, unroll, pf, c.dev, (int)tab.size(), grid, b->tc, s, L));
       double bytes = 0.0;
       for (Job *j : kv.second) {
         const int active = std::min(L, j->d.t0 + j->d.steps - b->t);
-        bytes += (double)active * (20.0 * j->H->col.size() + 4.0 * (j->n + 1) + 48.0 * j->R * (double)j->n);
+        bytes += (double)active * step_bytes(*j);
       }
       LQ_TRY(time_end(ctx, kCatSpmv, ev, bytes, L));
       if (timing) {
@@ -283,7 +294,7 @@ int run_chunk(lq_batch b) {
           tu.best = kUnrolls[bi];
         }
       }
-      LQ_TRY(launch_batch_reduce(ctx->stream, c.dev, (int)tab.size(), b->tc, L, kp));
+      LQ_TRY(launch_batch_reduce(ctx->stream, c.dev, (int)tab.size(), b->tc, L));
     }
     LQ_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     b->t += L;

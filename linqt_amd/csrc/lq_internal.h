@@ -175,7 +175,7 @@ struct BatchJobDev {
   double2 *buf0, *buf1;  // T_s ring
   double2 *partial;      // [chunk slot][nblk][k-width] dot partials
   double2 *mom;          // [M][k-width] per-state moments
-  int n, k, t0, steps, blk0, nblk;
+  int n, k, kp, t0, steps, blk0, nblk;  // kp: k padded to a power of two
 };
 
 // Launchers (lq_spmv.hip).  Return LQ_OK or an error code.
@@ -195,9 +195,10 @@ int launch_copy(hipStream_t st, double2 *dst, const double2 *src, size_t count);
 // Batched recursion (one width class kp, grid = sum of the jobs' nblk): step
 // slot of the chunk of nslots steps whose first launch index is *tc.
 // equal_slices: every job in dictionary form has slices of one width.
-int launch_spmm_batch(hipStream_t st, int kp, int unroll, const BatchJobDev *jobs, int njobs, int grid,
-                      const int *tc, int slot, int nslots, bool equal_slices);
-int launch_batch_reduce(hipStream_t st, const BatchJobDev *jobs, int njobs, const int *tc, int nslots, int kp);
+int launch_spmm_batch(hipStream_t st, int unroll, bool pf, const BatchJobDev *jobs, int njobs, int grid, const int *tc,
+                      int slot, int nslots);
+bool spmm_batch_pf(int kp, bool equal_slices);  // whether jobs of this width can run with pf
+int launch_batch_reduce(hipStream_t st, const BatchJobDev *jobs, int njobs, const int *tc, int nslots);
 int launch_set_int(hipStream_t st, int *p, int v);
 // dst[i*g + v] = src[(r0 + v)*n + i] (state-major device states -> [n][g]).
 int launch_interleave(hipStream_t st, const double2 *src, int n, int r0, int g, double2 *dst);

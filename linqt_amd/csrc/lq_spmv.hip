@@ -64,9 +64,8 @@ __device__ __forceinline__ void block_reduce_store(const double2 *d, double2 (*s
 // The nd (0..3) moments of a kDotPhi step: the step's own to partial, the ones
 // before it to the slots before, slot values apart.
 template <int KP>
-__device__ __forceinline__ void store_phi_dots(const double2 *d, int nd, double2 *partial, long long slot,
-                                               long long block) {
-  __shared__ double2 sh[3][256];
+__device__ __forceinline__ void store_phi_dots(const double2 *d, int nd, double2 (*sh)[256], double2 *partial,
+                                               long long slot, long long block) {
   if (nd == 1)
     block_reduce_store<KP, 1>(d, sh, partial, 0, block);
   else if (nd == 2)
@@ -495,29 +494,25 @@ __global__ __launch_bounds__(256) void k_spmm(int n, MatArgs m, double2 alpha, d
     __shared__ double2 sh[2][256];
     block_reduce_store<KP, 2>(d, sh, partial, KP, (long long)blockIdx.x * 2 * KP);
   }
-  if constexpr (DOT == kDotPhi)
-    store_phi_dots<KP>(d, fa.nd, partial, (long long)gridDim.x * KP, (long long)blockIdx.x * KP);
+  if constexpr (DOT == kDotPhi) {
+    __shared__ double2 sh[3][256];
+    store_phi_dots<KP>(d, fa.nd, sh, partial, (long long)gridDim.x * KP, (long long)blockIdx.x * KP);
+  }
 }
 
-// Batched recursion step over many independent jobs (one vector-width class):
-// block b belongs to the job j with blk0_j <= b < blk0_j + nblk_j and runs that
-// job's step s = t - t0_j with the same row schedule, dot fusion and partial
-// layout as a single-job launch with nblk_j blocks, so every job's moments are
-// independent of what else is in the batch.
+// Batched recursion step over many independent jobs: block b belongs to the job
+// j with blk0_j <= b < blk0_j + nblk_j and runs that job's step s = t - t0_j with
+// the same row schedule, dot fusion and partial layout as a single-job launch with
+// nblk_j blocks, so every job's moments are independent of what else is in the
+// batch.
 //   s == 0:  T_1 = H~ T_0                     (x = buf0, y = buf1)
 //   s >= 1:  T_{s+1} = 2 H~ T_s - T_{s-1}     (in place over T_{s-1})
-template <int KP, int kUnroll, bool PF = false>
-__global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restrict__ jobs, int njobs,
-                                                    const int *__restrict__ tc, int slot, int nslots, int ntz) {
-  int lo = 0, hi = njobs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (jobs[mid].blk0 <= (int)blockIdx.x) lo = mid;
-    else hi = mid - 1;
-  }
-  const BatchJobDev &J = jobs[lo];
-  const int s = tc[0] + slot - J.t0;
-  if (s < 0 || s >= J.steps) return;  // whole block leaves together
+// The jobs of one launch may have any vector widths: a block takes its job's by a
+// branch that is the same for all its lanes, and all widths share one set of LDS
+// arrays.
+template <int KP, int kUnroll, bool PF>
+__device__ __forceinline__ void batch_step(const BatchJobDev &J, int s, int slot, int nslots, int ntz, double2 *sdict,
+                                           int2 *sgeo, double2 (*sh)[256]) {
   const int lb = blockIdx.x - J.blk0;
   SetArgs sa{};
   const bool odd = s & 1;
@@ -538,8 +533,6 @@ __global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restric
   bf.nd = __builtin_amdgcn_readfirstlane(
       slot % 3 == 2 || slot == nslots - 1 || s == J.steps - 1 ? min(slot % 3, s) + 1 : 0);
   if (J.ndict > 0) {
-    __shared__ double2 sdict[256];
-    __shared__ int2 sgeo[PF ? kPfGroups : 1];
     const double2 tv = table_value(J.dict, J.ndict);  // J is the same for the whole block
     auto staged = [&]() {
       sdict[threadIdx.x] = tv;
@@ -563,14 +556,41 @@ __global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restric
     spmm_body<KP, kDotPhi, kUnroll, PlainMat>(J.n, mat, alpha, beta, sa, groups, J.phi, lb, J.nblk, d, bf, nullptr,
                                               [] {});
   }
-  store_phi_dots<KP>(d, bf.nd, J.partial + (size_t)slot * J.nblk * KP, (long long)J.nblk * KP, (long long)lb * KP);
+  store_phi_dots<KP>(d, bf.nd, sh, J.partial + (size_t)slot * J.nblk * KP, (long long)J.nblk * KP, (long long)lb * KP);
+}
+
+template <int kUnroll, bool PF>
+__global__ __launch_bounds__(256) void k_spmm_batch(const BatchJobDev *__restrict__ jobs, int njobs,
+                                                    const int *__restrict__ tc, int slot, int nslots, int ntz) {
+  __shared__ double2 sdict[256];
+  __shared__ int2 sgeo[PF ? kPfGroups : 1];
+  __shared__ double2 sh[3][256];
+  int lo = 0, hi = njobs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].blk0 <= (int)blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const BatchJobDev &J = jobs[lo];
+  const int s = tc[0] + slot - J.t0;
+  if (s < 0 || s >= J.steps) return;  // whole block leaves together
+  switch (J.kp) {
+    case 1: batch_step<1, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 2: batch_step<2, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 4: batch_step<4, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 8: batch_step<8, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 16: batch_step<16, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 32: batch_step<32, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+    case 64: batch_step<64, kUnroll, PF>(J, s, slot, nslots, ntz, sdict, sgeo, sh); break;
+  }
 }
 
 // mom[(s + 1) * KP + v] = sum_b partial[slot][b][v] for every step s a job ran
 // in this chunk (the same summation order as k_reduce_partials).
 __global__ __launch_bounds__(256) void k_batch_reduce(const BatchJobDev *__restrict__ jobs,
-                                                      const int *__restrict__ tc, int nslots, int kp) {
+                                                      const int *__restrict__ tc, int nslots) {
   const BatchJobDev &J = jobs[blockIdx.y];
+  const int kp = J.kp;
   const int slot = blockIdx.x;
   const int s = tc[0] + slot - J.t0;
   if (s < 0 || s >= J.steps) return;  // uniform over the block
@@ -980,44 +1000,35 @@ int launch_spmm(hipStream_t st, const SellDev &A, double2 alpha, double2 beta, c
   }
 }
 
-int launch_spmm_batch(hipStream_t st, int kp, int unroll, const BatchJobDev *jobs, int njobs, int grid,
-                      const int *tc, int slot, int nslots, bool equal_slices) {
+bool spmm_batch_pf(int kp, bool equal_slices) { return (256 / kp <= 64 || equal_slices) && spmm_pf(); }
+
+int launch_spmm_batch(hipStream_t st, int unroll, bool pf, const BatchJobDev *jobs, int njobs, int grid, const int *tc,
+                      int slot, int nslots) {
   if (njobs <= 0 || grid <= 0) return LQ_OK;
   // T_{n-1} loaded non-temporally: the batch mix holds jobs whose vector
   // blocks exceed the MALL (0.8 % faster over the mix); LQ_SPMM_NT=0 turns it off
   static const int ntz = env_int("LQ_SPMM_NT", 1) >= 1 ? 1 : 0;
-#define LQ_BU(KPV, UV)                                                                                        \
-  if (kp == KPV && unroll == UV) {                                                                          \
-    if ((256 / KPV <= 64 || equal_slices) && spmm_pf())                                                     \
-      hipLaunchKernelGGL((k_spmm_batch<KPV, UV, true>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot, \
-                         nslots, ntz);                                                                      \
-    else                                                                                                    \
-      hipLaunchKernelGGL((k_spmm_batch<KPV, UV>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot,      \
-                         nslots, ntz);                                                                      \
-    LQ_HIP_CHECK(hipGetLastError());                                                                        \
-    return LQ_OK;                                                                                           \
+#define LQ_BU(UV)                                                                                                     \
+  if (unroll == UV) {                                                                                                 \
+    if (pf)                                                                                                           \
+      hipLaunchKernelGGL((k_spmm_batch<UV, true>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot, nslots, ntz); \
+    else                                                                                                              \
+      hipLaunchKernelGGL((k_spmm_batch<UV, false>), dim3(grid), dim3(256), 0, st, jobs, njobs, tc, slot, nslots, ntz); \
+    LQ_HIP_CHECK(hipGetLastError());                                                                                  \
+    return LQ_OK;                                                                                                     \
   }
-#define LQ_BK(KPV) LQ_BU(KPV, 4) LQ_BU(KPV, 8) LQ_BU(KPV, 12) LQ_BU(KPV, 16)
-  LQ_BK(1)
-  LQ_BK(2)
-  LQ_BK(4)
-  LQ_BK(8)
-  LQ_BK(16)
-  LQ_BK(32)
-  LQ_BK(64)
-#undef LQ_BK
+  LQ_BU(4)
+  LQ_BU(8)
+  LQ_BU(12)
+  LQ_BU(16)
 #undef LQ_BU
-  set_error("launch_spmm_batch: unsupported width %d / unroll %d", kp, unroll);
+  set_error("launch_spmm_batch: unsupported unroll %d", unroll);
   return LQ_ERR_ARG;
 }
 
-int launch_batch_reduce(hipStream_t st, const BatchJobDev *jobs, int njobs, const int *tc, int nslots, int kp) {
+int launch_batch_reduce(hipStream_t st, const BatchJobDev *jobs, int njobs, const int *tc, int nslots) {
   if (njobs <= 0 || nslots <= 0) return LQ_OK;
-  if (kp <= 0 || kp > 256 || (kp & (kp - 1))) {
-    set_error("launch_batch_reduce: width %d is not a power of two <= 256", kp);
-    return LQ_ERR_ARG;
-  }
-  hipLaunchKernelGGL(k_batch_reduce, dim3(nslots, njobs), dim3(256), 0, st, jobs, tc, nslots, kp);
+  hipLaunchKernelGGL(k_batch_reduce, dim3(nslots, njobs), dim3(256), 0, st, jobs, tc, nslots);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }
