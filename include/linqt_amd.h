@@ -306,7 +306,7 @@ int lq_linear_grid(lq_ctx ctx, int kind, const double *mu, int M0, int M1, int n
 /* ---- batched spectral-moment jobs ------------------------------------------ */
 /* Many SpectralMoments jobs (OP = identity, src/chebyshev_solver.cpp:176-200),
  * each with its own rescaled H, states and M, advanced together: one grouped
- * launch per recursion step per vector-width class.  This is the submit/poll
+ * launch per recursion step for all vector widths.  This is the submit/poll
  * surface a serving loop drives (continuous batching): jobs submitted between
  * lq_batch_run calls join at the next chunk boundary when their device
  * footprint fits the budget.  A job's moments are bitwise identical alone,

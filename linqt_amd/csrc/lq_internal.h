@@ -192,7 +192,7 @@ int launch_dot(hipStream_t st, int n, int k, const double2 *a, const double2 *b,
 int launch_reduce_partials(hipStream_t st, const double2 *partial, int nslots, int grid, int width,
                            double2 *out);
 int launch_copy(hipStream_t st, double2 *dst, const double2 *src, size_t count);
-// Batched recursion (one width class kp, grid = sum of the jobs' nblk): step
+// Batched recursion (jobs of any widths, grid = sum of the jobs' nblk): step
 // slot of the chunk of nslots steps whose first launch index is *tc.
 // equal_slices: every job in dictionary form has slices of one width.
 int launch_spmm_batch(hipStream_t st, int unroll, bool pf, const BatchJobDev *jobs, int njobs, int grid, const int *tc,
