@@ -132,9 +132,22 @@ struct NbScal {
   int state, it, i;
 };
 
+// Power of two of a's larger component (0 for zero, infinities and NaN).
+__device__ __forceinline__ int scale_of(double2 a) {
+  const double m = fmax(fabs(a.x), fabs(a.y));
+  return m > 0.0 && m < HUGE_VAL ? ilogb(m) : 0;
+}
+__device__ __forceinline__ double2 scaled(double2 a, int e) { return make_double2(ldexp(a.x, e), ldexp(a.y, e)); }
+
+// a / b with both brought to the size of 1 by powers of two: the solver's scalars
+// grow with |b|^2 of the system, so the square of a divisor would leave the
+// exponent's range for right-hand sides beyond 1e-77 .. 1e77.
 __device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
+  const int ea = scale_of(a), eb = scale_of(b);
+  a = scaled(a, -ea);
+  b = scaled(b, -eb);
   const double m = b.x * b.x + b.y * b.y;
-  return make_double2((a.x * b.x + a.y * b.y) / m, (a.y * b.x - a.x * b.y) / m);
+  return scaled(make_double2((a.x * b.x + a.y * b.y) / m, (a.y * b.x - a.x * b.y) / m), ea - eb);
 }
 
 // Every thread: (sum, sum) of nblk pairs (NV = 2) or single values of partials, in
