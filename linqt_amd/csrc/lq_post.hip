@@ -352,71 +352,96 @@ __device__ __forceinline__ double lin_xgrid(int kind, int i, int num_div) {
   return -xb + i * (2 * xb) / (num_div - 1);
 }
 
-// One block per energy i = step * block, the sums as written above.  step = 1,
-// every energy: Spectral, BastinII and small tables.  step = num_div - 1, the two
-// end points of the others, where x = +-1 makes every coefficient infinite and
-// the printed NaN or infinity is the one the sources' order of operations gives.
+// Blocks of kLinE energies, the sums as written above: every energy of the tools
+// Spectral, BastinII, Sea and of small tables (ends = num_div), else the first and
+// last `ends` energies, see k_grid_energies.  x = +-1 makes every coefficient
+// infinite, and the printed NaN or infinity is the one the sources' order of
+// operations gives.  Two energies share a reading of the table, which is what the
+// sums wait for (M = 512: 4 MB from L2 for each block).
+template <int KIND>
+constexpr int kLinE = KIND == 0 || KIND == 4 ? 1 : 2;
+
 template <int KIND>
 __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1, int num_div,
-                                                       int step, double scale, double *__restrict__ kern) {
-  extern __shared__ double2 lv[];  // left vector(s): [M0] (BastinII: [2][M0])
-  const int i = blockIdx.x * step;
-  const double x = lin_xgrid(KIND, i, num_div);
+                                                       int ends, int count, double scale, double *__restrict__ kern) {
+  extern __shared__ double2 lv[];  // left vector(s): [M0] (BastinII: [2][M0]; two energies in x and y)
+  constexpr int kE = kLinE<KIND>;
+  int i[kE];
+  double x[kE];
+#pragma unroll
+  for (int e = 0; e < kE; ++e) {
+    const int t = min((int)blockIdx.x * kE + e, count - 1);
+    i[e] = t < ends ? t : num_div - count + t;
+    x[e] = lin_xgrid(KIND, i[e], num_div);
+  }
   for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) {
     if (KIND == 4) {
-      lv[m0] = greenR_chebF(x, m0);
-      lv[M0 + m0] = DgreenR_chebF(x, m0);
+      lv[m0] = greenR_chebF(x[0], m0);
+      lv[M0 + m0] = DgreenR_chebF(x[0], m0);
     } else if (KIND == 5) {
-      lv[m0] = make_double2(greenR_chebF(x, m0).y, 0.0);
+      lv[m0] = make_double2(greenR_chebF(x[0], m0).y, greenR_chebF(x[kE - 1], m0).y);
     } else {
-      lv[m0] = make_double2(delta_chebF(x, m0), 0.0);
+      lv[m0] = make_double2(delta_chebF(x[0], m0), delta_chebF(x[kE - 1], m0));
     }
   }
   __syncthreads();
-  double acc = 0;
+  double acc[kE] = {};
   if (KIND == 0) {
-    for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) acc += lv[m0].x * mu[m0].x;
+    for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) acc[0] += lv[m0].x * mu[m0].x;
   } else {
     for (int m1 = threadIdx.x; m1 < M1; m1 += blockDim.x) {
-      double zr = 0, zi = 0, wr = 0, wi = 0;
+      double zr[kE] = {}, zi[kE] = {}, wr = 0, wi = 0;
       for (int m0 = 0; m0 < M0; ++m0) {
         const double2 v = mu[(size_t)m0 * M1 + m1];
         const double2 l = lv[m0];
         if (KIND == 4) {
-          zr += l.x * v.x - l.y * v.y;
-          zi += l.x * v.y + l.y * v.x;
+          zr[0] += l.x * v.x - l.y * v.y;
+          zi[0] += l.x * v.y + l.y * v.x;
           const double2 dl = lv[M0 + m0];
           wr += dl.x * v.x - dl.y * v.y;
           wi += dl.x * v.y + dl.y * v.x;
         } else {
-          zr = fma(l.x, v.x, zr);
-          zi = fma(l.x, v.y, zi);
+#pragma unroll
+          for (int e = 0; e < kE; ++e) {
+            zr[e] = fma(e ? l.y : l.x, v.x, zr[e]);
+            zi[e] = fma(e ? l.y : l.x, v.y, zi[e]);
+          }
         }
       }
-      if (KIND == 1 || KIND == 3) {
-        const double2 g = greenR_chebF(x, m1);
-        acc += g.x * zi + g.y * zr;  // Im(g z)
-      } else if (KIND == 2) {
-        const double2 g = DgreenR_chebF(x, m1);
-        acc += g.x * zi + g.y * zr;
-      } else if (KIND == 6) {
-        acc += delta_chebF(x, m1) * zr;
-      } else if (KIND == 5) {
-        acc += 4.0 * DgreenR_chebF(x, m1).x * zi;
-      } else {  // 4: -Re(DgR z_gR - gR z_DgR)
-        const double2 d = DgreenR_chebF(x, m1), g = greenR_chebF(x, m1);
-        acc += -((d.x * zr - d.y * zi) - (g.x * wr - g.y * wi));
+#pragma unroll
+      for (int e = 0; e < kE; ++e) {
+        if (KIND == 1 || KIND == 3) {
+          const double2 g = greenR_chebF(x[e], m1);
+          acc[e] += g.x * zi[e] + g.y * zr[e];  // Im(g z)
+        } else if (KIND == 2) {
+          const double2 g = DgreenR_chebF(x[e], m1);
+          acc[e] += g.x * zi[e] + g.y * zr[e];
+        } else if (KIND == 6) {
+          acc[e] += delta_chebF(x[e], m1) * zr[e];
+        } else if (KIND == 5) {
+          acc[e] += 4.0 * DgreenR_chebF(x[e], m1).x * zi[e];
+        } else {  // 4: -Re(DgR z_gR - gR z_DgR)
+          const double2 d = DgreenR_chebF(x[e], m1), g = greenR_chebF(x[e], m1);
+          acc[e] += -((d.x * zr[e] - d.y * zi[e]) - (g.x * wr - g.y * wi));
+        }
       }
     }
   }
-  __shared__ double red[256];
-  red[threadIdx.x] = acc;
+  __shared__ double red[kE][256];
+#pragma unroll
+  for (int e = 0; e < kE; ++e) red[e][threadIdx.x] = acc[e];
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    if (threadIdx.x < s) {
+#pragma unroll
+      for (int e = 0; e < kE; ++e) red[e][threadIdx.x] += red[e][threadIdx.x + s];
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) kern[i] = red[0] * scale;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int e = 0; e < kE; ++e) kern[i[e]] = red[e][0] * scale;
+  }
 }
 
 // The same sums through the table's diagonal sums U (k_diag_grid): with
@@ -424,16 +449,17 @@ __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict
 //   C1 = sum cos m0 cos m1 Re mu = sum_q U0 cos q theta,  S1 = sum cos m0 sin m1 Im mu = sum U1 sin,
 //   C2 = sum m1 cos m0 cos m1 Im mu = sum U2 cos,         S2 = sum m1 cos m0 sin m1 Re mu = sum U3 sin,
 //   Greenwood, BastinI  -(C1 + S1) / (pi f^2);   Surf  C1 / (pi f)^2;
-//   Bastin  [f (C2 - S2) - x (C1 + S1)] / (pi f^4);  Sea  -4 [f C2 - x S1] / f^4.
-// One wavefront for kEw energies (the U of a lane's q are loaded once for all).
-// The angle is taken from the nearer band edge, theta' = acos |x|, with the
-// parity of q for x < 0: the phases' rounding q theta' 2^-53 then is smallest
-// towards the edges, where 1/f^4 magnifies it.
+//   Bastin  [f (C2 - S2) - x (C1 + S1)] / (pi f^4).
+// One wavefront for kEw energies (the U of a lane's q are loaded once for all), i
+// from `ends` to num_div - ends: towards the band ends the sums over one index
+// nearly cancel and 1/f^4 magnifies what is left of U's rounding, so there the
+// double sums are formed as written (k_linear_kernel).  The phase q theta' is
+// reduced with its rounding (theta' = acos |x|, with the parity of q for x < 0).
 constexpr int kEw = 4;
 template <int KIND>
-__global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__ seq, int Q,
-                                                      int num_div, double scale, double *__restrict__ kern) {
-  const int l = threadIdx.x, i0 = blockIdx.x * kEw;
+__global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__ seq, int Q, int num_div, int ends,
+                                                      double scale, double *__restrict__ kern) {
+  const int l = threadIdx.x, i0 = ends + blockIdx.x * kEw;
   double x[kEw], th[kEw], u[kEw], v[kEw];
 #pragma unroll
   for (int e = 0; e < kEw; ++e) {
@@ -446,8 +472,10 @@ __global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__
     const double4 w = *(const double4 *)(seq + 4 * (size_t)q);
 #pragma unroll
     for (int e = 0; e < kEw; ++e) {
-      double sn, cs;
-      sincos(q * th[e], &sn, &cs);
+      const double ph = q * th[e], lo = fma((double)q, th[e], -ph);
+      double s0, c0;
+      sincos(ph, &s0, &c0);
+      double sn = fma(c0, lo, s0), cs = fma(-s0, lo, c0);
       if (x[e] < 0.0) {  // q theta = q pi - q theta'
         if (q & 1)
           cs = -cs;
@@ -457,9 +485,6 @@ __global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__
       // u: the sum without the weight m1, v: the weighted one
       if (KIND == 6) {
         u[e] = fma(w.x, cs, u[e]);
-      } else if (KIND == 5) {
-        u[e] = fma(w.y, sn, u[e]);
-        v[e] = fma(w.z, cs, v[e]);
       } else {
         u[e] = fma(w.x, cs, fma(w.y, sn, u[e]));
         if (KIND == 2) v[e] = fma(w.z, cs, fma(-w.w, sn, v[e]));
@@ -473,15 +498,11 @@ __global__ __launch_bounds__(64) void k_grid_energies(const double *__restrict__
       v[e] += __shfl_down(v[e], d);
     }
     const int i = i0 + e;
-    // the linear grid's end points belong to k_linear_kernel (x = +-1; not Bastin's)
-    const bool end = KIND != 2 && (i == 0 || i == num_div - 1);
-    if (l == 0 && i < num_div && !end) {
+    if (l == 0 && i < num_div - ends) {
       const double f2 = 1.0 - x[e] * x[e], f = sqrt(f2);
       double r;
       if (KIND == 6)
         r = u[e] / f2 / (kPi * kPi);
-      else if (KIND == 5)
-        r = -4.0 * (f * v[e] - x[e] * u[e]) / f2 / f2;
       else if (KIND == 2)
         r = (f * v[e] - x[e] * u[e]) / f2 / f2 / kPi;
       else
@@ -599,19 +620,21 @@ int launch_diag_sums(hipStream_t st, const double2 *mu, int ld, int M0, int M1, 
   return LQ_OK;
 }
 
-// kern[i] of a grid tool (kinds as k_grid_energies) from the table's diagonal sums.
-int launch_grid_kernel(hipStream_t st, int kind, const double2 *mu, int M0, int M1, int num_div, double scale,
+// kern[i], ends <= i < num_div - ends, of a grid tool (kinds as k_grid_energies)
+// from the table's diagonal sums.
+int launch_grid_kernel(hipStream_t st, int kind, const double2 *mu, int M0, int M1, int num_div, int ends, double scale,
                        double2 *diag, double *kern) {
   const int Q = M0 + M1 - 1;
   LQ_TRY(launch_diag_sums(st, mu, M1, M0, M1, nullptr, 1, diag));
   double *seq = (double *)(diag + (size_t)4 * Q * diag_chunks(M0));
   hipLaunchKernelGGL(k_diag_grid, dim3((Q + 63) / 64), dim3(64), 0, st, diag, diag_chunks(M0), M0, M1, seq);
-  const dim3 grid((num_div + kEw - 1) / kEw);
+  const dim3 grid((num_div - 2 * ends + kEw - 1) / kEw);
   switch (kind) {
 #define LQ_GE(K) \
-  case K: hipLaunchKernelGGL((k_grid_energies<K>), grid, dim3(64), 0, st, seq, Q, num_div, scale, kern); break;
-    LQ_GE(1) LQ_GE(2) LQ_GE(5) LQ_GE(6)
-    case 3: hipLaunchKernelGGL((k_grid_energies<1>), grid, dim3(64), 0, st, seq, Q, num_div, scale, kern); break;
+  hipLaunchKernelGGL((k_grid_energies<K>), grid, dim3(64), 0, st, seq, Q, num_div, ends, scale, kern)
+    case 1: case 3: LQ_GE(1); break;
+    case 2: LQ_GE(2); break;
+    case 6: LQ_GE(6); break;
 #undef LQ_GE
   }
   LQ_HIP_CHECK(hipGetLastError());
@@ -653,24 +676,33 @@ int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int 
     set_error("launch_linear_grid: %d moments exceed the LDS table (max %d)", M0, kind == 4 ? 2048 : 4096);
     return LQ_ERR_UNSUPPORTED;
   }
-  // Through the diagonal sums from 64 x 64 moments on: 0.12 ms instead of 2.28 at
-  // M = 512 (15360 energies), and there 4e-14 from exact sums instead of 3e-13;
-  // below, the direct sums take a few microseconds and are as near (M = 40 x 65,
-  // Bastin: 8e-15 instead of 2e-14).
-  const bool diagonal = kind != 0 && kind != 4 && (long long)M0 * M1 >= 4096;
-  auto direct = [&](auto kernel) {
-    const bool ends = diagonal;
-    hipLaunchKernelGGL(kernel, dim3(ends ? 2 : num_div), dim3(256), lds, st, mu, M0, M1, num_div,
-                       ends ? num_div - 1 : 1, scale, kern);
+  // Through the diagonal sums from 64 x 64 moments on; below, the double sums take a
+  // few microseconds.  Energies with |x| > 0.9 are left to the double sums.  Damped
+  // tables of 64 to 512 orders with levels inside (-0.93, 0.93), largest error against
+  // 80-bit sums over the curve's largest value, double / diagonal sums: |x| < 0.9
+  // 2e-15 .. 6e-13 / 2e-16 .. 4e-15, but 0.97 < |x| < 0.99 (Bastin) 8e-16 .. 2e-14 /
+  // 4e-15 .. 2e-13 and beyond 0.998 (Greenwood, Surf) 1e-15 .. 1e-13 / 4e-15 .. 3e-13.
+  // Sea stays with the double sums throughout: its running sum begins with the NaN of
+  // x = -1, so no printed value could show an error of another form.
+  const bool diagonal = (kind == 1 || kind == 2 || kind == 3 || kind == 6) && (long long)M0 * M1 >= 4096;
+  const double xb = kind == 2 ? 0.99 : 1.0;
+  const int most = (num_div + 1) / 2;
+  const int ends = diagonal ? std::max(1, std::min(most, (int)((xb - 0.9) / (2 * xb) * (num_div - 1)) + 1)) : num_div;
+  const int count = std::min(num_div, 2 * ends);
+  auto direct = [&](auto kernel, int per) {
+    hipLaunchKernelGGL(kernel, dim3((count + per - 1) / per), dim3(256), lds, st, mu, M0, M1, num_div, ends, count, scale,
+                       kern);
   };
-  if (diagonal) LQ_TRY(launch_grid_kernel(st, kind, mu, M0, M1, num_div, scale, diag, kern));
+  if (diagonal && count < num_div) LQ_TRY(launch_grid_kernel(st, kind, mu, M0, M1, num_div, ends, scale, diag, kern));
   switch (kind) {
-    case 0: direct(k_linear_kernel<0>); break;
-    case 1: case 3: direct(k_linear_kernel<1>); break;
-    case 2: if (!diagonal) direct(k_linear_kernel<2>); break;  // its grid ends inside (-1, 1)
-    case 4: direct(k_linear_kernel<4>); break;
-    case 5: direct(k_linear_kernel<5>); break;
-    case 6: direct(k_linear_kernel<6>); break;
+#define LQ_LIN(K) direct(k_linear_kernel<K>, kLinE<K>)
+    case 0: LQ_LIN(0); break;
+    case 1: case 3: LQ_LIN(1); break;
+    case 2: LQ_LIN(2); break;
+    case 4: LQ_LIN(4); break;
+    case 5: LQ_LIN(5); break;
+    case 6: LQ_LIN(6); break;
+#undef LQ_LIN
   }
   hipLaunchKernelGGL(k_linear_columns, dim3((num_div + 63) / 64), dim3(64), 0, st, kind, num_div, a, Ec, kern, E, out);
   if (kind == 2 || kind == 4 || kind == 5)

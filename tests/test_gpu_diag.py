@@ -1,7 +1,9 @@
 """Energy-grid sums through a table's diagonals: the linear-grid tools on both
 sides of the size from which they are used (64 x 64 moments), square and not,
 and the Kubo sums of small tables (up to 128 orders), against the oracle.
-Tolerance 1e-9 of the largest value, as for every energy grid."""
+Tolerance 1e-9 of the largest value, as for every energy grid.  Kind 5 (Sea)
+prints a running sum that begins with the NaN of x = -1: only its energies and
+the NaN can be compared."""
 import numpy as np
 import pytest
 
@@ -25,6 +27,7 @@ def test_linear_grid_by_diagonals(ctx, oracle, kind, M0, M1, nd):
     assert np.allclose(E, Eo, rtol=0, atol=1e-13)
     assert np.array_equal(np.isnan(v), np.isnan(vo)) and np.array_equal(np.isinf(v), np.isinf(vo))
     fin = np.isfinite(vo)
+    assert fin.sum() == 0 if kind == 5 else fin.sum() >= len(vo) - 2
     if fin.any():
         assert rel_inf(v[fin], vo[fin]) < 1e-9
 
