@@ -1406,21 +1406,30 @@ int run_pipe2d(Pipe2D &P, const double *phi, int R) {
 }
 
 // Kubo energy sums from transforms of the stored vectors (lq_kubosum.hip)
-// instead of the moment table.  Times at 262144 elements, Bastin, sums against
-// table (without the table's own energy sums, 6 M^2 flop at 70 TFLOP/s over
-// whole 128 x 128 tiles), one operator / two:
-//   M =  128: 1.27 / 1.68 ms against 0.37 / 0.74: up to there the table;
-//   M =  200: 1.41 / 1.84 against 1.47 / 2.95;  512: 2.56 / 3.39 against 5.9 / 11.8;
-//   M =  513 .. 640: 9.1 .. 10.1 / 11.3 .. 12.6 against 9.2 / 18.4 (three
-//   frequency sets that each read the vectors): the table for one operator;
-//   M =  700: 10.4 / 12.9 against 13.3 / 26.5;  1024: 15.4 / 19.9 against 23.6 / 47.
+// instead of the moment table, for K = n R stored elements of an order.  Both
+// sides measured, sums / table, with what follows them up to 1024 energies, in ms,
+// Bastin (Greenwood: the table's times, the sums' 0.6 to 1.0 of these):
+//            one operator                             two operators
+//   M        K = 512      18432        262088         512          18432        262088
+//   100      .029 / .056  .108 / .106  1.13 / .60     .034 / .104  .142 / .203  1.52 / 1.20
+//   128      .029 / .071  .108 / .092  1.12 / .44     .034 / .134  .141 / .176  1.55 / .88
+//   129      .031 / .073  .112 / .161  1.11 / 1.53    .035 / .137  .142 / .310  1.56 / 3.03
+//   256      .034 / .080  .119 / .184  1.25 / 1.61    .038 / .150  .152 / .355  1.71 / 3.16
+//   512      .051 / .102  .211 / .544  2.42 / 6.05    .065 / .189  .282 / 1.07  3.27 / 11.8
+//   513      .069 / .106  .605 / .840  9.13 / 9.47    .102 / .197  .797 / 1.67  11.3 / 18.8
+//   640      .073 / .112  .642 / .883  10.1 / 9.58    .105 / .203  .886 / 1.74  12.6 / 18.9
+//   1024     .102 / .187  .825 / 1.98  15.3 / 23.6    .149 / .341  1.19 / 3.94  20.0 / 46.8
+// Up to M = 128, one tile of the contraction, the table is the faster one for many
+// elements (M = 24: six times), and what the sums would save for few is below 0.1 ms
+// of a solve: the table.  Above it the sums, but for one operator at M = 513 .. 640
+// (three frequency sets that each read the vectors) from 2^17 elements on.
 // LQ_KUBO=table keeps the table.
-bool kubo_by_sums(int M, int nopr) {
+bool kubo_by_sums(int M, int nopr, long long K) {
   static const bool off = [] {
     const char *e = getenv("LQ_KUBO");
     return e && strcmp(e, "table") == 0;
   }();
-  return !off && M > 128 && (M <= 512 || M > 640 || nopr > 1) && kubosum_supported(M);
+  return !off && M > 128 && (M <= 512 || M > 640 || nopr > 1 || K < (1 << 17)) && kubosum_supported(M);
 }
 
 int ord_of(int p, int B) { return (p / B) * (B - 1) + (p % B); }
@@ -2309,7 +2318,7 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
   double2 *raw, *fd, *tables = nullptr, *seq = nullptr;
   double *coef;
   KuboSums sums{formula, nullptr, nullptr, nullptr};
-  const bool use_sums = precision == LQ_PREC_FP64 && kubo_by_sums(M, nopr);
+  const bool use_sums = precision == LQ_PREC_FP64 && kubo_by_sums(M, nopr, (long long)n * R);
   if (M > 4096) {
     set_error("lq_kubo_fft: M = %d exceeds 4096", M);
     for (auto m : owned) lq_csr_destroy(m);

@@ -30,7 +30,7 @@ def _ops(ctx, oracle, L):
     (1, 129, 130, 3, 1, 1, 1), (0, 129, 258, 3, 3, 2, 1), (1, 255, 255, 4, 1, 2, 1), (1, 256, 300, 3, 1, 3, 1),
     (0, 257, 514, 3, 1, 1, 1), (1, 300, 301, 5, 1, 2, 5), (1, 512, 512, 3, 2, 2, 1), (0, 512, 1024, 3, 1, 3, 1),
     (1, 513, 513, 3, 1, 2, 1), (1, 641, 700, 3, 1, 1, 1), (0, 768, 768, 3, 1, 2, 1), (1, 769, 800, 3, 1, 1, 1),
-    (1, 1030, 1030, 3, 1, 1, 1), (1, 200, 200, 3, 33, 2, 1)])
+    (1, 1030, 1030, 3, 1, 1, 1), (1, 200, 200, 3, 33, 2, 1), (1, 513, 513, 3, 2, 1, 1), (0, 640, 640, 4, 1, 1, 1)])
 def test_kubo_sums_vs_oracle(ctx, oracle, formula, M, nump, L, R, nopr, ns):
     print("[case] kubo sums", formula, M, nump, L, R, nopr, ns, flush=True)
     n, G, O = _ops(ctx, oracle, L)
