@@ -356,13 +356,17 @@ __device__ __forceinline__ double lin_xgrid(int kind, int i, int num_div) {
 // Spectral, BastinII, Sea and of small tables (ends = num_div), else the first and
 // last `ends` energies, see k_grid_energies.  x = +-1 makes every coefficient
 // infinite, and the printed NaN or infinity is the one the sources' order of
-// operations gives.  Two energies share a reading of the table, which is what the
-// sums wait for (M = 512: 4 MB from L2 for each block).
+// operations gives.  The sums wait for the table (4 MB from L2 for each block at
+// M = 512): two energies share a reading, 16 rows are on their way at a time, and
+// blocks of 512 threads are all resident (256 threads: a last round of few blocks).
+// 620 energies at M = 512: 133 us, with 256 threads 250.
 template <int KIND>
 constexpr int kLinE = KIND == 0 || KIND == 4 ? 1 : 2;
+template <int KIND>
+constexpr int kLinT = KIND == 0 || KIND == 4 ? 256 : 512;
 
 template <int KIND>
-__global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1, int num_div,
+__global__ __launch_bounds__(kLinT<KIND>) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1, int num_div,
                                                        int ends, int count, double scale, double *__restrict__ kern) {
   extern __shared__ double2 lv[];  // left vector(s): [M0] (BastinII: [2][M0]; two energies in x and y)
   constexpr int kE = kLinE<KIND>;
@@ -391,6 +395,7 @@ __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict
   } else {
     for (int m1 = threadIdx.x; m1 < M1; m1 += blockDim.x) {
       double zr[kE] = {}, zi[kE] = {}, wr = 0, wi = 0;
+#pragma unroll 16
       for (int m0 = 0; m0 < M0; ++m0) {
         const double2 v = mu[(size_t)m0 * M1 + m1];
         const double2 l = lv[m0];
@@ -427,11 +432,11 @@ __global__ __launch_bounds__(256) void k_linear_kernel(const double2 *__restrict
       }
     }
   }
-  __shared__ double red[kE][256];
+  __shared__ double red[kE][kLinT<KIND>];
 #pragma unroll
   for (int e = 0; e < kE; ++e) red[e][threadIdx.x] = acc[e];
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
+  for (int s = kLinT<KIND> / 2; s > 0; s >>= 1) {
     if (threadIdx.x < s) {
 #pragma unroll
       for (int e = 0; e < kE; ++e) red[e][threadIdx.x] += red[e][threadIdx.x + s];
@@ -677,25 +682,26 @@ int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int 
     return LQ_ERR_UNSUPPORTED;
   }
   // Through the diagonal sums from 64 x 64 moments on; below, the double sums take a
-  // few microseconds.  Energies with |x| > 0.9 are left to the double sums.  Damped
+  // few microseconds.  Energies with |x| > 0.95 are left to the double sums.  Damped
   // tables of 64 to 512 orders with levels inside (-0.93, 0.93), largest error against
-  // 80-bit sums over the curve's largest value, double / diagonal sums: |x| < 0.9
-  // 2e-15 .. 6e-13 / 2e-16 .. 4e-15, but 0.97 < |x| < 0.99 (Bastin) 8e-16 .. 2e-14 /
-  // 4e-15 .. 2e-13 and beyond 0.998 (Greenwood, Surf) 1e-15 .. 1e-13 / 4e-15 .. 3e-13.
+  // 80-bit sums over the curve's largest value, double / diagonal sums: |x| < 0.95
+  // 2e-15 .. 6e-13 / 3e-16 .. 3e-14 (never the larger one), but 0.97 < |x| < 0.99
+  // (Bastin) 8e-16 .. 2e-14 / 4e-15 .. 2e-13 and beyond 0.998 (Greenwood, Surf)
+  // 1e-15 .. 1e-13 / 4e-15 .. 3e-13.
   // Sea stays with the double sums throughout: its running sum begins with the NaN of
   // x = -1, so no printed value could show an error of another form.
   const bool diagonal = (kind == 1 || kind == 2 || kind == 3 || kind == 6) && (long long)M0 * M1 >= 4096;
   const double xb = kind == 2 ? 0.99 : 1.0;
   const int most = (num_div + 1) / 2;
-  const int ends = diagonal ? std::max(1, std::min(most, (int)((xb - 0.9) / (2 * xb) * (num_div - 1)) + 1)) : num_div;
+  const int ends = diagonal ? std::max(1, std::min(most, (int)((xb - 0.95) / (2 * xb) * (num_div - 1)) + 1)) : num_div;
   const int count = std::min(num_div, 2 * ends);
-  auto direct = [&](auto kernel, int per) {
-    hipLaunchKernelGGL(kernel, dim3((count + per - 1) / per), dim3(256), lds, st, mu, M0, M1, num_div, ends, count, scale,
+  auto direct = [&](auto kernel, int per, int threads) {
+    hipLaunchKernelGGL(kernel, dim3((count + per - 1) / per), dim3(threads), lds, st, mu, M0, M1, num_div, ends, count, scale,
                        kern);
   };
   if (diagonal && count < num_div) LQ_TRY(launch_grid_kernel(st, kind, mu, M0, M1, num_div, ends, scale, diag, kern));
   switch (kind) {
-#define LQ_LIN(K) direct(k_linear_kernel<K>, kLinE<K>)
+#define LQ_LIN(K) direct(k_linear_kernel<K>, kLinE<K>, kLinT<K>)
     case 0: LQ_LIN(0); break;
     case 1: case 3: LQ_LIN(1); break;
     case 2: LQ_LIN(2); break;
