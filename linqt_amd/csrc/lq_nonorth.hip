@@ -15,8 +15,8 @@
 // |r|^2 and <r0|r>.  The kernels that need a dot product's value sum the partials
 // of the blocks before them, every block for itself, in one fixed order; the
 // stopping test is theirs too, and an iteration queued past it leaves the vectors
-// alone.  So the host queues as many iterations as the solve before took and only
-// then looks (one small copy), where a copy and a wait for each of three dot
+// alone.  So the host queues as many iterations as the solve before took, at most
+// 16, and only then looks (one small copy), where a copy and a wait for each of three dot
 // products had taken most of an iteration's 100 us (N = 16380, 147 iterations in
 // 49 solves: 15.1 -> 5.5 ms; what is left is launches of 4 to 5 us).
 #include <algorithm>
@@ -30,6 +30,10 @@ namespace {
 
 constexpr int kNbThreads = 256;
 constexpr int kNbBlocks = 512;
+// Most iterations queued before the host looks.  A look costs half an iteration's
+// launches; an iteration queued past the end costs all of them and its two products,
+// which test no state (a load before their first one took 4 % of a solve).
+constexpr int kNbQueue = 16;
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -368,7 +372,7 @@ struct Bicg {
     LQ_HIP_CHECK(hipGetLastError());
     // i numbers the iterations queued (rho is stored by its parity); the count that
     // maxit bounds starts anew at the first restart, as the sources' does
-    int i = 0, base = 0, restarts = 0, queue = expect + 1;
+    int i = 0, base = 0, restarts = 0, queue = 1 + std::min(kNbQueue, expect);
     bool first = true, resumed = false;
     auto rest = [&]() -> int {  // iteration i after its k_nb_p
       LQ_TRY(apply_S(y, v, kDotPhi, r0));
@@ -404,7 +408,7 @@ struct Bicg {
       } else {  // the last test went on
         LQ_TRY(rest());
         ++i;
-        queue = 1 + std::min(8, (i - base) / 4);
+        queue = 1 + std::min(kNbQueue, (i - base) / 4);
       }
     }
     iterations += host->it;
