@@ -867,7 +867,7 @@ struct Pipe2D {
   int nopr;
   const lq_csr *OPR;
   int n, ML, MR;
-  double2 *raw;  // nopr tables of ML x MR (ld MR)
+  double2 *raw;  // nopr tables of ML x MR (ld MR); null with sums: taken when the streamed pipeline runs
   int precision = LQ_PREC_FP64;
   const KuboSums *sums = nullptr;
   bool summed = false;
@@ -1394,6 +1394,8 @@ int run_pipe2d(Pipe2D &P, const double *phi, int R) {
     }
     return LQ_OK;
   }
+  if (!P.raw)
+    LQ_TRY(ctx_buf(P.ctx, "raw", (size_t)P.ML * P.MR * P.nopr * sizeof(double2), (void **)&P.raw));
   int g = 1;
   StreamPlan pl;
   LQ_TRY(stream_plan(P.ctx, R, P.n, P.ML, P.MR, P.nopr, P.precision, &g, &pl));
@@ -2315,7 +2317,7 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
     }
   }
   const size_t tab = (size_t)M * M;
-  double2 *raw, *fd, *tables = nullptr, *seq = nullptr;
+  double2 *raw = nullptr, *fd, *tables = nullptr, *seq = nullptr;
   double *coef;
   KuboSums sums{formula, nullptr, nullptr, nullptr};
   const bool use_sums = precision == LQ_PREC_FP64 && kubo_by_sums(M, nopr, (long long)n * R);
@@ -2325,7 +2327,7 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
     return LQ_ERR_ARG;
   }
   const size_t count = kubosum_spec_count(M, formula, nopr);
-  int rc = ctx_buf(ctx, "raw", tab * nopr * sizeof(double2), (void **)&raw);
+  int rc = use_sums ? LQ_OK : ctx_buf(ctx, "raw", tab * nopr * sizeof(double2), (void **)&raw);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_fd", (size_t)2 * nump * nopr * sizeof(double2), (void **)&fd);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_coef", (size_t)M * sizeof(double), (void **)&coef);
   if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_seq", count * sizeof(double2), (void **)&seq);
@@ -2362,7 +2364,7 @@ int lq_kubo_fft(lq_csr H, lq_csr OPL, int nopr, const lq_csr *OPR, const double 
       double2 *diag;
       if (rc == LQ_OK) rc = ctx_buf(ctx, "kubo_diag", diag_bytes(M, M), (void **)&diag);
       for (int o = 0; o < nopr && rc == LQ_OK; ++o)
-        rc = launch_diag_kubo(ctx->stream, raw + o * tab, M, coef, formula, 1.0 / R, kubosum_length(M), diag,
+        rc = launch_diag_kubo(ctx->stream, P.raw + o * tab, M, coef, formula, 1.0 / R, kubosum_length(M), diag,
                               seq + o * (count / nopr));
     }
     if (rc == LQ_OK) rc = launch_kubo_energies(ctx->stream, formula, seq, M, nopr, nump, fd);

@@ -7,6 +7,8 @@ Tolerance 1e-10 of the largest value, as for every Kubo sum: both sides round
 each of the O(M) terms of a site to 1e-16 of its size and the oracle's angles
 m theta to m 1e-16, which leaves about M 1e-16 <= 1e-13.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -40,3 +42,21 @@ def test_kubo_sums_vs_oracle(ctx, oracle, formula, M, nump, L, R, nopr, ns):
     for o in range(nopr):
         ref, _ = oracle.kubo_fft(O[0], O[1], oops[o], phi, M, nump, formula, num_sections=ns)
         assert rel_inf(got[o], ref) < 1e-10, o
+
+
+def test_no_table_is_allocated(oracle):
+    """The sums take the place of the moment tables, so a solve of two operators at
+    2048 orders and few elements stays below the tables' 134 MB of device memory."""
+    print("[case] memory of the sums", flush=True)
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    c = lq.Context(0)
+    n, G, _ = _ops(c, oracle, 3)
+    phi = lattices.random_phase_states(n, 1, seed=7)
+    lq.kubo_fft(G[0], G[1], [G[1], G[2]], phi, 200, 2048, 1)  # the device's own first allocations
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    lq.kubo_fft(G[0], G[1], [G[1], G[2]], phi, 2048, 2048, 1)
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    assert before - free.value < 2 * 2048 * 2048 * 16
+    c.close()
