@@ -1347,7 +1347,9 @@ int stream_plan(lq_ctx ctx, int R, int n, int ML, int MR, int nopr, int precisio
   const size_t vb = (size_t)n * sizeof(double2);                       // one vector of one state
   const size_t rbuf = (size_t)pl->nbuf * nopr * pl->BR + 5;             // right buffers, phi, ring, carry
   const size_t planes = precision_int8(precision) ? (size_t)2 * precision * n : 0;  // digit bytes per row
-  const size_t work = (size_t)512 * 128 * 128 * sizeof(double2);       // split-K partial tables (about)
+  // split-K partial tables: at most 1024 tiles of 128 x 128 (the other precisions and
+  // the 64 x 64 kernel: fewer elements), or 8 of the whole block
+  const size_t work = ((size_t)1024 * 128 * 128 + (size_t)8 * ML * std::min(nopr, 2) * pl->BR) * sizeof(double2);
   const size_t budget = pipe_budget(ctx);
   auto per_state = [&](size_t BL) { return (BL + rbuf) * vb + (BL + 2 * pl->BR) * planes; };
   size_t g = budget > work ? (budget - work) / per_state(ML) : 0;

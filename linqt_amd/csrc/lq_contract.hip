@@ -888,8 +888,10 @@ bool t128_fits(long long lda, long long ldb) {
 // same chunks in the same order and gives the same tables.
 // Against chunks of at least 4096 elements and no look at the last round (us,
 // contraction + reduction): 100 x 100 x 8192 602 -> 36, 128 x 128 x 8192
-// 1438 -> 49, 300 x 300 x 54150 1484 -> 729, 512 x 512 x 8192 1450 -> 211; tables
-// with K in the millions keep their chunks.
+// 1438 -> 49, 300 x 300 x 54150 1484 -> 729, 512 x 512 x 8192 1450 -> 211.
+// At K = 2^21 tables of 128 to 256, of 512 and of 1024 square keep the chunks they
+// had; others have more (below 128: 256 -> 512, 300: 40 -> 56, 640: 16 -> 40, 768:
+// 8 -> 24), up to 1024 tiles in all.
 constexpr int kMinChunk = 64;
 int choose_nsplit(int M0, int M1, long long K) {
   const long long by_k = std::max(1LL, K / kMinChunk);
