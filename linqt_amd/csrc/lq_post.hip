@@ -356,20 +356,24 @@ __device__ __forceinline__ double lin_xgrid(int kind, int i, int num_div) {
 // Spectral, BastinII, Sea and of small tables (ends = num_div), else the first and
 // last `ends` energies, see k_grid_energies.  x = +-1 makes every coefficient
 // infinite, and the printed NaN or infinity is the one the sources' order of
-// operations gives.  The sums wait for the table (4 MB from L2 for each block at
-// M = 512): two energies share a reading, 16 rows are on their way at a time, and
-// blocks of 512 threads are all resident (256 threads: a last round of few blocks).
-// 620 energies at M = 512: 133 us, with 256 threads 250.
+// operations gives.  What bounds them is the wait for the table's rows, 4 MB a block
+// at M = 512: the energies of a block share a reading, eight rows are on their way
+// at a time (the compiler waits for each row where the batch may end early), and
+// all blocks are resident.  620 energies at M = 512, Bastin: 51 us; two energies
+// 73; two and one row at a time 133, with 256 threads 250.
 template <int KIND>
-constexpr int kLinE = KIND == 0 || KIND == 4 ? 1 : 2;
+constexpr int kLinE = KIND == 0 || KIND == 4 ? 1 : 4;
+constexpr int kLinRows = 8;
 template <int KIND>
 constexpr int kLinT = KIND == 0 || KIND == 4 ? 256 : 512;
 
 template <int KIND>
-__global__ __launch_bounds__(kLinT<KIND>) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1, int num_div,
-                                                       int ends, int count, double scale, double *__restrict__ kern) {
-  extern __shared__ double2 lv[];  // left vector(s): [M0] (BastinII: [2][M0]; two energies in x and y)
+__global__ __launch_bounds__(kLinT<KIND>) void k_linear_kernel(const double2 *__restrict__ mu, int M0, int M1,
+                                                               int num_div, int ends, int count, double scale,
+                                                               double *__restrict__ kern) {
+  extern __shared__ double2 lv[];  // left vectors: [M0][kE] doubles (BastinII: [2][M0] complex)
   constexpr int kE = kLinE<KIND>;
+  double *lx = (double *)lv;
   int i[kE];
   double x[kE];
 #pragma unroll
@@ -382,37 +386,44 @@ __global__ __launch_bounds__(kLinT<KIND>) void k_linear_kernel(const double2 *__
     if (KIND == 4) {
       lv[m0] = greenR_chebF(x[0], m0);
       lv[M0 + m0] = DgreenR_chebF(x[0], m0);
-    } else if (KIND == 5) {
-      lv[m0] = make_double2(greenR_chebF(x[0], m0).y, greenR_chebF(x[kE - 1], m0).y);
     } else {
-      lv[m0] = make_double2(delta_chebF(x[0], m0), delta_chebF(x[kE - 1], m0));
+#pragma unroll
+      for (int e = 0; e < kE; ++e) lx[m0 * kE + e] = KIND == 5 ? greenR_chebF(x[e], m0).y : delta_chebF(x[e], m0);
     }
   }
   __syncthreads();
   double acc[kE] = {};
   if (KIND == 0) {
-    for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) acc[0] += lv[m0].x * mu[m0].x;
+    for (int m0 = threadIdx.x; m0 < M0; m0 += blockDim.x) acc[0] += lx[m0] * mu[m0].x;
   } else {
     for (int m1 = threadIdx.x; m1 < M1; m1 += blockDim.x) {
       double zr[kE] = {}, zi[kE] = {}, wr = 0, wi = 0;
-#pragma unroll 16
-      for (int m0 = 0; m0 < M0; ++m0) {
-        const double2 v = mu[(size_t)m0 * M1 + m1];
-        const double2 l = lv[m0];
+      auto add = [&](int m0, double2 v) {
         if (KIND == 4) {
+          const double2 l = lv[m0], dl = lv[M0 + m0];
           zr[0] += l.x * v.x - l.y * v.y;
           zi[0] += l.x * v.y + l.y * v.x;
-          const double2 dl = lv[M0 + m0];
           wr += dl.x * v.x - dl.y * v.y;
           wi += dl.x * v.y + dl.y * v.x;
         } else {
 #pragma unroll
           for (int e = 0; e < kE; ++e) {
-            zr[e] = fma(e ? l.y : l.x, v.x, zr[e]);
-            zi[e] = fma(e ? l.y : l.x, v.y, zi[e]);
+            const double l = lx[m0 * kE + e];
+            zr[e] = fma(l, v.x, zr[e]);
+            zi[e] = fma(l, v.y, zi[e]);
           }
         }
+      };
+      int m0 = 0;
+      for (; m0 + kLinRows <= M0; m0 += kLinRows) {
+        double2 row[kLinRows];
+#pragma unroll
+        for (int u = 0; u < kLinRows; ++u) row[u] = mu[(size_t)(m0 + u) * M1 + m1];
+        __builtin_amdgcn_sched_barrier(0);  // all on their way before the first is used
+#pragma unroll
+        for (int u = 0; u < kLinRows; ++u) add(m0 + u, row[u]);
       }
+      for (; m0 < M0; ++m0) add(m0, mu[(size_t)m0 * M1 + m1]);
 #pragma unroll
       for (int e = 0; e < kE; ++e) {
         if (KIND == 1 || KIND == 3) {
@@ -676,9 +687,9 @@ int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int 
       set_error("launch_linear_grid: unknown kind %d", kind);
       return LQ_ERR_ARG;
   }
-  const size_t lds = sizeof(double2) * (size_t)M0 * (kind == 4 ? 2 : 1);
-  if (lds > 64 * 1024) {
-    set_error("launch_linear_grid: %d moments exceed the LDS table (max %d)", M0, kind == 4 ? 2048 : 4096);
+  const int most_orders = kind == 4 ? 2048 : 4096;
+  if (M0 > most_orders) {
+    set_error("launch_linear_grid: %d moments exceed the LDS table (max %d)", M0, most_orders);
     return LQ_ERR_UNSUPPORTED;
   }
   // Through the diagonal sums from 64 x 64 moments on; below, the double sums take a
@@ -695,13 +706,16 @@ int launch_linear_grid(hipStream_t st, int kind, const double2 *mu, int M0, int 
   const int most = (num_div + 1) / 2;
   const int ends = diagonal ? std::max(1, std::min(most, (int)((xb - 0.95) / (2 * xb) * (num_div - 1)) + 1)) : num_div;
   const int count = std::min(num_div, 2 * ends);
-  auto direct = [&](auto kernel, int per, int threads) {
-    hipLaunchKernelGGL(kernel, dim3((count + per - 1) / per), dim3(threads), lds, st, mu, M0, M1, num_div, ends, count, scale,
-                       kern);
+  auto direct = [&](auto kernel, int per, int threads) -> int {
+    const size_t lds = kind == 4 ? sizeof(double2) * 2 * (size_t)M0 : sizeof(double) * per * (size_t)M0;
+    LQ_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kernel, dim3((count + per - 1) / per), dim3(threads), lds, st, mu, M0, M1, num_div, ends, count,
+                       scale, kern);
+    return LQ_OK;
   };
   if (diagonal && count < num_div) LQ_TRY(launch_grid_kernel(st, kind, mu, M0, M1, num_div, ends, scale, diag, kern));
   switch (kind) {
-#define LQ_LIN(K) direct(k_linear_kernel<K>, kLinE<K>, kLinT<K>)
+#define LQ_LIN(K) LQ_TRY(direct(k_linear_kernel<K>, kLinE<K>, kLinT<K>))
     case 0: LQ_LIN(0); break;
     case 1: case 3: LQ_LIN(1); break;
     case 2: LQ_LIN(2); break;
@@ -800,7 +814,8 @@ int launch_greenwood_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, 
   return LQ_OK;
 }
 
-int launch_bastin_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, int n, double W, double Ec, int num_div, double *scratch, double *E, double *out) {
+int launch_bastin_fftgrid(hipStream_t st, const double2 *mu, int M0, int M1, int n, double W, double Ec, int num_div,
+                          double *scratch, double *E, double *out) {
   double *energies = scratch, *kern = scratch + num_div;
   const size_t lds = sizeof(double) * (size_t)M0;
   if (lds > 64 * 1024) {
