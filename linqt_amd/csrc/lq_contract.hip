@@ -988,8 +988,8 @@ int launch_contract_f64(hipStream_t st, const double2 *A, long long lda, int M0,
 int launch_contract_reduce(hipStream_t st, const double2 *work, int nsplit, int M0, int M1, double2 *out, int ldo,
                            int accumulate) {
   const long long total = (long long)M0 * M1;
-  hipLaunchKernelGGL(k_contract_reduce, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st, work, nsplit, M0,
-                     M1, out, ldo, accumulate);
+  hipLaunchKernelGGL(k_contract_reduce, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st, work,
+                     nsplit, M0, M1, out, ldo, accumulate);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }
@@ -1001,8 +1001,8 @@ int launch_contract_reduce_cols(hipStream_t st, const double2 *work, int nsplit,
     return LQ_ERR_ARG;
   }
   const long long total = (long long)M0 * M1;
-  hipLaunchKernelGGL(k_contract_reduce_cols, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st, work, nsplit,
-                     M0, M1, bc, outs[0], M1 / bc > 1 ? outs[1] : outs[0], ldo, accumulate);
+  hipLaunchKernelGGL(k_contract_reduce_cols, dim3((unsigned)((total + kRedElems - 1) / kRedElems)), dim3(256), 0, st,
+                     work, nsplit, M0, M1, bc, outs[0], M1 / bc > 1 ? outs[1] : outs[0], ldo, accumulate);
   LQ_HIP_CHECK(hipGetLastError());
   return LQ_OK;
 }

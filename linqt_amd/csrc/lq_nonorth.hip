@@ -179,9 +179,9 @@ __device__ __forceinline__ void sum_partials(const double2 *__restrict__ partial
   if (NV == 2) b = sh[1][0];
 }
 
-// Iteration i (the count-th that maxit bounds): the stopping test, rho and beta; then p = r + beta (p - w v), y =
-// dinv p.  partial: of |r|^2 and <r0|r> (first: of |b|^2).  resumed: after a
-// restart, rho and the test are settled.
+// Iteration i (the count-th that maxit bounds): the stopping test, rho and beta;
+// then p = r + beta (p - w v), y = dinv p.  partial: of |r|^2 and <r0|r> (first: of
+// |b|^2).  resumed: after a restart, rho and the test are settled.
 __global__ __launch_bounds__(kNbThreads) void k_nb_p(int n, int i, int count, int first, int resumed, double tol,
                                                       int maxit, const double2 *__restrict__ partial, int nblk,
                                                       NbScal *sc,
