@@ -635,6 +635,12 @@ def main():
                                "TFLOP/s": tm["contract_flops"] / launches / (avg_ms * 1e-3) / 1e12}
         config["moments_basis"] = ("2 M^2 R a step, the moments of the tables; the energy sums are formed from the "
                                    "stored vectors without them, so moments/s is an equivalent rate")
+    if args.workload == "bastin" and args.precision != "fp64":
+        S = PRECISIONS[args.precision]
+        kernels["contract"] = {"ms_per_step": tm["contract_ms"] / tsteps,
+                               "launches_per_step": tm["contract_launches"] / tsteps,
+                               "kernel": f"k_contract_split<{S}>" if S in (2, 3) else f"k_contract_i8<{S}> + k_slice<{S}>",
+                               "complex_equiv_TFLOP/s": ctr_cplx_tfs}
     # HBM bytes per launch of the dominant kernel, from the committed PMC summary of this workload,
     # used only when it was measured on the kernel sources of this tree
     traffic_tab = {}
